@@ -15,6 +15,7 @@
 #include "../../include/bhsparse_spmv.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstdint>
 #include <cstring>
@@ -30,6 +31,13 @@
 // reaches it only through the address scratch_ptr() looks up.
 constexpr size_t kScratchBytes = size_t(8) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+
+// Words of the rows that cross logical waves (bhs::ChainBuf), for the calls of
+// the allocation-free entry points that run as one kernel: up to kChainWaves
+// logical waves.  Their own array: between calls no other call writes it.
+constexpr int kChainWaves = 1 << 16;
+constexpr size_t kChainBytes = 16 + 8 + 8 + 8;   // per logical wave
+static __device__ __align__(256) unsigned char chain_scratch[kChainBytes * kChainWaves];
 
 namespace {
 
@@ -75,6 +83,11 @@ constexpr long long kMaxNnz = 0x7fffffffLL - 4 * kMaxTile;
 
 enum ValueKind { kFloat = 1, kDouble = 2 };
 
+// How the plain segmented sum runs: a wave walking its tiles, then
+// calibrate_kernel; a wave per tile, then calibrate_kernel; or a wave per tile
+// that also finishes the rows crossing logical waves (one kernel in all).
+enum SegsumKernel { kWaveLoop, kTilePerWave, kTilePerWaveFused };
+
 template <typename T>
 struct Impl {
     int device = -1;
@@ -118,9 +131,13 @@ struct Impl {
     int chunk_parts = 2;   // row chunk of the segmented sum: 2 or 4 parts of 64 rows
     int *d_tile_row = nullptr;
     int tile_cap = 0;
+    // one buffer for sync_cap logical waves: bhs::ChainBuf's words, sync_val, sync_row
+    unsigned char *d_waves = nullptr;
     int *d_sync_row = nullptr;
     T *d_sync_val = nullptr;
     int sync_cap = 0;
+    SegsumKernel kernel = kWaveLoop;
+    unsigned call = 0;                  // number of the last fused launch
 
     unsigned long long *d_counters = nullptr;   // 8 x u64 scratch for stats/features
     T *d_floor = nullptr;                       // per-lane partials of the floor probe
@@ -132,7 +149,8 @@ struct Impl {
     // ev[0]/ev[2]: recorded around a whole call; ev[1]/ev[3]: attached to the
     // main kernel's dispatch (hipExtLaunchKernelGGL), its exact duration
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    size_t max_lds = 65536;   // per-block LDS limit of the device
+    size_t max_lds = 65536;   // per-block LDS limit of a configuration
+    size_t dev_lds = 65536;   // per-block LDS limit of the device
 };
 
 struct HandleBox {
@@ -180,7 +198,7 @@ int create(bhs_handle_t *h)
     return BHSPARSE_SUCCESS;
 }
 
-int scratch_ptr(void **out);
+int scratch_ptr(void *(&out)[2]);
 
 template <typename T>
 int init_platform(bhs_handle_t h, int device)
@@ -200,6 +218,7 @@ int init_platform(bhs_handle_t h, int device)
         return set_error(BHSPARSE_INVALID_ARGUMENT, "handle already bound to another device");
     BHS_HIP(hipSetDevice(device));
     im->max_lds = std::min<size_t>(prop.sharedMemPerBlock, 65536);
+    im->dev_lds = prop.sharedMemPerBlock;
     if (!im->platform) {
         BHS_HIP(hipStreamCreateWithFlags(&im->stream, hipStreamNonBlocking));
         for (auto &e : im->ev) BHS_HIP(create_timing_event(&e));
@@ -207,8 +226,8 @@ int init_platform(bhs_handle_t h, int device)
     }
     im->device = device;
     im->platform = true;
-    void *sp = nullptr;              // the device's scratch address, looked up once
-    return scratch_ptr(&sp);
+    void *sp[2];                     // the device's scratch addresses, looked up once
+    return scratch_ptr(sp);
 }
 
 // Frees an array allocated by alloc_data in `mode`.
@@ -235,8 +254,9 @@ void release_data(Impl<T> *im)
     free_data(im->d_x, im->data_mode);
     free_data(im->d_y, im->data_mode);
     free_ptr(im->d_tile_row);
-    free_ptr(im->d_sync_row);
-    free_ptr(im->d_sync_val);
+    free_ptr(im->d_waves);
+    im->d_sync_row = nullptr;
+    im->d_sync_val = nullptr;
     free_ptr(im->d_floor);
     free_ptr(im->d_prow_ptr);
     free_ptr(im->d_pcol);
@@ -245,6 +265,7 @@ void release_data(Impl<T> *im)
     free_ptr(im->d_pmask);
     free_ptr(im->d_pbase);
     free_ptr(im->d_chains);
+    im->kernel = kWaveLoop;
     im->chain_cap = 0;
     im->h_prow_ptr = {};
     im->h_prow_of = {};
@@ -509,6 +530,60 @@ int build_chains(Impl<T> *im, long long PW, long long NW)
     return BHSPARSE_SUCCESS;
 }
 
+// Waves of a block of the one-wave-per-tile kernel: whole logical waves.
+inline int tile_block_waves(const bhs_config &c)
+{
+    return c.waves_per_block % c.tiles_per_wave == 0 ? c.waves_per_block : c.tiles_per_wave;
+}
+
+template <typename T>
+size_t tile_lds_bytes(int S, int waves)
+{
+    return (size_t)waves * (64 * (size_t)S * sizeof(T) + 256) + sizeof(bhs::TileShare<T>);
+}
+
+// The kernel of the plain layout, by shape and number of logical waves NW (y
+// is the same bits in all three).  Whole calls in us, loop / one wave per tile /
+// the same fused, cold caches:
+//  * T = 4, S = 8, fp64: 65,536 uniform rows (NW 513) 17.1 / 13.7 / 11.4; 7-point
+//    Laplacian 100^3 (3.4k) 34.8 / 30.2 / 27.8; power law, 10M nonzeros (4.9k)
+//    118.8 / 114.9 / 112.7; Laplacian 160^3 (14k) 110 / 104 / 102; 3x3 blocks, 54M
+//    (26k) 167 / 164 / 163, warm 160 / 153 / 153.  The fused end of a wave (an
+//    exchange past the L2s) is cheaper than a launch of calibrate_kernel until
+//    the device is full of waves for many rounds: up to 16,384.
+//  * T = 1 is one wave per tile anyway; only the fused end gains: S = 8, 65,536
+//    rows (2k) 13.2 -> 11.8, band of 27 (16k) 29.5 -> 26.8, Laplacian 160^3 (56k)
+//    102 -> 104.  S = 4 has half the work per exchange: 65,536 rows (4.1k) 13.4 ->
+//    12.4, 2M-nonzero power law (7.8k) 22.2 -> 22.7: up to 4,096.
+//  * fp32, S = 4 (2 KB of A a wave), T = 4, Laplacian 160^3: 63.9 / 70.8 warm.
+//  * T > 1 with up to 32 logical waves (65,000 nonzeros at the default tile)
+//    stays on the loop, 14 us against 6: the fixed default tile is the yardstick
+//    of the tuner's speedup (at least 1.2 over its test set), and what such a
+//    matrix should run is the tuner's csr-vector (4.4 us) or one tile per wave.
+// Shapes the one-wave-per-tile kernel is not built for (T not a power of two
+// up to 8, S = 32) and blocks beyond the device's LDS take the loop.
+template <typename T>
+SegsumKernel pick_kernel(const Impl<T> *im, long long NW)
+{
+    const bhs_config &c = im->cfg;
+    const int TPW = c.tiles_per_wave, S = c.items_per_lane;
+    if (c.variant != BHS_VARIANT_SEGSUM || S > 16 || TPW > bhs::kMaxGroup || (TPW & (TPW - 1)))
+        return kWaveLoop;
+    if (tile_lds_bytes<T>(S, tile_block_waves(c)) > im->dev_lds) return kWaveLoop;
+    if (TPW > 1 && NW <= 32) return kWaveLoop;
+    if (NW <= (S == 4 ? 4096 : 16384)) return kTilePerWaveFused;
+    return TPW == 1 || S * sizeof(T) < 32 ? kWaveLoop : kTilePerWave;
+}
+
+// The words of ChainBuf for `waves` logical waves in one buffer of
+// waves * kChainBytes; `call` in 1 .. 2^31 - 1.
+inline bhs::ChainBuf chain_buf(unsigned char *p, long long waves, unsigned call)
+{
+    return {reinterpret_cast<unsigned long long *>(p),
+            reinterpret_cast<unsigned long long *>(p + 16 * waves), p + 24 * waves, p + 32 * waves,
+            call};
+}
+
 // Partition for the configured tile size and layout, and sizes of the
 // per-wave buffers.
 template <typename T>
@@ -529,12 +604,16 @@ int ensure_analysis(Impl<T> *im)
         im->tile_cap = (int)(NP + 1);
     }
     if (NW > im->sync_cap) {
-        free_ptr(im->d_sync_row);
-        free_ptr(im->d_sync_val);
-        BHS_HIP(hipMalloc(&im->d_sync_row, sizeof(int) * (size_t)std::max<long long>(NW, 1)));
-        BHS_HIP(hipMalloc(&im->d_sync_val, sizeof(T) * (size_t)std::max<long long>(NW, 1)));
-        im->sync_cap = (int)std::max<long long>(NW, 1);
+        free_ptr(im->d_waves);
+        im->sync_cap = 0;
+        BHS_HIP(hipMalloc(&im->d_waves, (kChainBytes + sizeof(T) + sizeof(int)) * (size_t)NW));
+        im->d_sync_val = reinterpret_cast<T *>(im->d_waves + kChainBytes * NW);
+        im->d_sync_row = reinterpret_cast<int *>(im->d_sync_val + NW);
+        im->sync_cap = (int)NW;
+        launch_fill(im, reinterpret_cast<unsigned long long *>(im->d_waves),
+                    (long long)kChainBytes / 8 * NW);      // all words empty
     }
+    im->kernel = pick_kernel(im, NW);
     const int threads = 256;
     const int blocks = (int)((NP + 1 + threads - 1) / threads);
     if (L.rows > 0)
@@ -682,7 +761,7 @@ template <typename T, int S, bool STATS, int CP>
 void launch_segsum_s(Impl<T> *im, T alpha, unsigned long long *stats, hipEvent_t e0, hipEvent_t e1)
 {
     const Layout<T> L = active_layout(im);
-    bhs::SegsumParams<T> q;
+    bhs::SegsumParams<T> q{};
     q.m = L.rows;
     q.nnz = im->nnz;
     q.NP = im->NP;
@@ -699,8 +778,8 @@ void launch_segsum_s(Impl<T> *im, T alpha, unsigned long long *stats, hipEvent_t
     const size_t lds = (size_t)q.wpb * q.wave_lds_bytes;
     // the stacked matrix of the column-panel layout has no empty rows
     auto kern = im->cfg.variant == BHS_VARIANT_SEGSUM_PANELS
-                    ? bhs::segsum_kernel<T, S, STATS, CP, false, true>
-                    : bhs::segsum_kernel<T, S, STATS, CP, false, false>;
+                    ? bhs::segsum_kernel<T, S, STATS, CP, true>
+                    : bhs::segsum_kernel<T, S, STATS, CP, false>;
     if (e0 && e1)
         hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(64 * q.wpb), (std::uint32_t)lds, im->stream,
                               e0, e1, 0u, L.row_ptr, L.col, L.val, (const T *)im->d_x, L.y,
@@ -710,6 +789,55 @@ void launch_segsum_s(Impl<T> *im, T alpha, unsigned long long *stats, hipEvent_t
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * q.wpb), lds, im->stream, L.row_ptr, L.col,
                            L.val, (const T *)im->d_x, L.y, (const int *)im->d_tile_row,
                            im->d_sync_row, im->d_sync_val, stats, q);
+}
+
+// One wave per tile (kTilePerWave, kTilePerWaveFused).
+template <typename T, int S, int CP>
+void launch_tiles_s(Impl<T> *im, T alpha, hipEvent_t e0, hipEvent_t e1)
+{
+    bhs::SegsumParams<T> q{};
+    q.m = im->m;
+    q.nnz = im->nnz;
+    q.NP = im->NP;
+    q.TPW = im->cfg.tiles_per_wave;
+    q.NW = im->NW;
+    q.lead_empty = im->lead_empty;
+    q.alpha = alpha;
+    const long long x_bytes = (long long)im->n * (long long)sizeof(T);
+    q.x_lines = x_bytes <= (1LL << 20) ? (x_bytes + 127) / 128 : 0;
+    q.x_far = x_bytes > 0xffffffffLL;
+    const int waves = tile_block_waves(im->cfg);
+    const bool fused = im->kernel == kTilePerWaveFused;
+    bhs::ChainBuf cb{};
+    if (fused) {
+        im->call = im->call < 0x7fffffffu ? im->call + 1 : 1;
+        cb = chain_buf(im->d_waves, im->sync_cap, im->call);
+    }
+    auto kern = fused ? bhs::segsum_tiles_kernel<T, S, CP, false, false, true>
+                      : bhs::segsum_tiles_kernel<T, S, CP, false, false, false>;
+    const dim3 grid((unsigned)((im->NP + waves - 1) / waves)), block(64 * waves);
+    const size_t lds = tile_lds_bytes<T>(S, waves);
+    if (e0 && e1)
+        hipExtLaunchKernelGGL(kern, grid, block, (std::uint32_t)lds, im->stream, e0, e1, 0u,
+                              (const int *)im->d_row_ptr, (const int *)im->d_col,
+                              (const T *)im->d_val, (const T *)im->d_x, im->d_y,
+                              (const int *)im->d_tile_row, im->d_sync_row, im->d_sync_val, cb, q);
+    else
+        hipLaunchKernelGGL(kern, grid, block, lds, im->stream, (const int *)im->d_row_ptr,
+                           (const int *)im->d_col, (const T *)im->d_val, (const T *)im->d_x,
+                           im->d_y, (const int *)im->d_tile_row, im->d_sync_row, im->d_sync_val,
+                           cb, q);
+}
+
+template <typename T>
+void launch_tiles(Impl<T> *im, T alpha, hipEvent_t e0, hipEvent_t e1)
+{
+    const bool wide = im->chunk_parts == 4;
+    switch (im->cfg.items_per_lane) {
+    case 4: wide ? launch_tiles_s<T, 4, 4>(im, alpha, e0, e1) : launch_tiles_s<T, 4, 2>(im, alpha, e0, e1); break;
+    case 8: wide ? launch_tiles_s<T, 8, 4>(im, alpha, e0, e1) : launch_tiles_s<T, 8, 2>(im, alpha, e0, e1); break;
+    default: wide ? launch_tiles_s<T, 16, 4>(im, alpha, e0, e1) : launch_tiles_s<T, 16, 2>(im, alpha, e0, e1); break;
+    }
 }
 
 template <typename T, bool STATS, int CP>
@@ -863,8 +991,10 @@ int enqueue_spmv(Impl<T> *im, T alpha, hipEvent_t main_start = nullptr,
     if (segsum_lds_bytes<T>(im->cfg) > im->max_lds)
         return set_error(BHSPARSE_INVALID_ARGUMENT,
                          "items_per_lane x waves_per_block needs more LDS than a block may use");
-    launch_segsum<T, false>(im, alpha, nullptr, main_start, main_done);
+    if (im->kernel == kWaveLoop) launch_segsum<T, false>(im, alpha, nullptr, main_start, main_done);
+    else launch_tiles(im, alpha, main_start, main_done);
     BHS_HIP(hipGetLastError());
+    if (im->kernel == kTilePerWaveFused) return BHSPARSE_SUCCESS;
     launch_calibrate(im);
     BHS_HIP(hipGetLastError());
     launch_combine(im);
@@ -1087,8 +1217,24 @@ int bench(bhs_handle_t h, T alpha, int warmup, int reps, long long flush_bytes, 
         BHS_HIP(hipEventElapsedTime(&a, im->ev[0], im->ev[2]));
         ms_total[i] = a;
     }
-    // the main kernel alone: events attached to its dispatch, separate calls
-    for (int i = 0; ms_main && i < reps; ++i) {
+    // the main kernel alone: events attached to its dispatch, separate calls.
+    // A call that is that one kernel is timed as a whole call: attached events
+    // add the write-back of what the flush left dirty in the caches (10.3 us
+    // against 7.2 us for 20,000 rows).
+    if (int rc = ensure_analysis(im)) return rc;
+    const bool one_kernel = im->cfg.variant == BHS_VARIANT_SEGSUM && im->NP > 0 &&
+                            im->kernel == kTilePerWaveFused;
+    for (int i = 0; ms_main && one_kernel && i < reps; ++i) {
+        flush();
+        BHS_HIP(hipEventRecord(im->ev[0], im->stream));
+        if (int rc = enqueue_spmv(im, alpha)) return rc;
+        BHS_HIP(hipEventRecord(im->ev[2], im->stream));
+        BHS_HIP(hipEventSynchronize(im->ev[2]));
+        float b = 0;
+        BHS_HIP(hipEventElapsedTime(&b, im->ev[0], im->ev[2]));
+        ms_main[i] = b;
+    }
+    for (int i = 0; ms_main && !one_kernel && i < reps; ++i) {
         flush();
         if (int rc = enqueue_spmv(im, alpha, im->ev[1], im->ev[3])) return rc;
         BHS_HIP(hipEventSynchronize(im->ev[3]));
@@ -1376,38 +1522,50 @@ int row_features(bhs_handle_t h, double *f)
 #include "bhs_batch.inc"
 
 // ---- y = alpha*A*x with no allocation ------------------------------------
-// Device scratch of the allocation-free entry point: the tile partition and
-// the waves' boundary-row partials, at most kScratchBytes.  One copy per
-// device, held until the process ends.  Host code never uses the array's
-// name as an address: scratch_ptr() looks the device's copy up once per
-// device (hipGetSymbolAddress, with that device current) and keeps it.
+// Device scratch of the allocation-free entry point: the words of the rows
+// that cross logical waves (chain_scratch) or, for matrices of more than
+// kChainWaves logical waves, the tile partition and the waves' boundary-row
+// partials (scratch, at most kScratchBytes).  One copy per device, held until
+// the process ends.  Host code never uses the arrays' names as addresses:
+// scratch_ptr() looks the device's copies up once per device
+// (hipGetSymbolAddress, with that device current) and keeps them.
 constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mu;
-void *g_scratch_dev[kScratchDevices] = {};
+void *g_scratch_dev[kScratchDevices][2] = {};
+std::atomic<unsigned> g_noalloc_call{0};   // number of the last one-kernel call
 
-// The current device's scratch (looked up on its first use on that device).
-int scratch_ptr(void **out)
+// The current device's {scratch, chain_scratch} (looked up on their first use
+// on that device).
+int scratch_ptr(void *(&out)[2])
 {
     int dev = -1;
     BHS_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= kScratchDevices)
         return set_error(BHSPARSE_UNSUPPORTED_DEVICE, "device index beyond the scratch table");
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_dev[dev]) {
-        void *p = nullptr;
+    if (!g_scratch_dev[dev][1]) {
+        void *p = nullptr, *c = nullptr;
         BHS_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-        if (!p) return set_error(BHSPARSE_HIP_ERROR, "hipGetSymbolAddress(scratch) gave null");
-        g_scratch_dev[dev] = p;
+        BHS_HIP(hipGetSymbolAddress(&c, HIP_SYMBOL(chain_scratch)));
+        if (!p || !c) return set_error(BHSPARSE_HIP_ERROR, "hipGetSymbolAddress(scratch) gave null");
+        g_scratch_dev[dev][0] = p;
+        g_scratch_dev[dev][1] = c;
     }
-    *out = g_scratch_dev[dev];
+    out[0] = g_scratch_dev[dev][0];
+    out[1] = g_scratch_dev[dev][1];
     return BHSPARSE_SUCCESS;
 }
 
-// The same kernels as a handle's default tile (segmented sum, S = 8, 4 waves
-// per block, 4 tiles per wave, plain layout): partition, segmented sum with
-// checked loads of the last tile (the caller's col/val are not padded),
-// calibration.  Enqueued on `stream`; nothing is allocated, copied to the
-// host or waited for, so a caller may capture it in a graph.
+// The sums of a handle's default tile (segmented sum, S = 8, 4 waves per
+// block, 4 tiles per wave, plain layout), one wave per tile, with checked loads
+// of the last tile (the caller's col/val are not padded).  Up to kChainWaves
+// logical waves (134M nonzeros) it is one kernel: each wave finds its rows by
+// itself and the rows crossing logical waves are finished where they end.
+// Whole passes, partition + kernel + calibration before, us: 8k nonzeros 13.9
+// -> 6.9, 1M (fp32) 19.2 -> 9.1, 2M power law 28.5 -> 19.4, 28M Laplacian 95.2
+// -> 82.7, 54M 3x3 blocks (fp32) 125 -> 115.  Beyond, the partition and the
+// calibration are launches of their own.  Enqueued on `stream`; nothing is
+// allocated, copied to the host or waited for, so a caller may capture it.
 template <typename T>
 int spmv_noalloc(int m, int n, int nnz, const int *row_ptr, const int *col, const T *val,
                  const T *x, T *y, T alpha, void *stream_v)
@@ -1433,46 +1591,53 @@ int spmv_noalloc(int m, int n, int nnz, const int *row_ptr, const int *col, cons
         return set_error(BHSPARSE_INVALID_ARGUMENT,
                          "matrix needs " + std::to_string(need) + " bytes of scratch, more than the " +
                              std::to_string(kScratchBytes) + " the allocation-free entry point has");
-    void *base = nullptr;
-    if (int rc = scratch_ptr(&base)) return rc;
-    unsigned char *sb = static_cast<unsigned char *>(base);
-    int *tile_row = reinterpret_cast<int *>(sb);
-    int *sync_row = reinterpret_cast<int *>(sb + o_sr);
-    T *sync_val = reinterpret_cast<T *>(sb + o_sv);
     const int threads = 256;
     if (NP == 0) {                                    // no nonzeros: y = 0
-        const long long blocks = std::min<long long>((m + threads - 1) / threads, 4096);
+        const long long blocks = std::min<long long>(((long long)m + threads - 1) / threads, 4096);
         hipLaunchKernelGGL(bhs::fill_kernel<T>, dim3((unsigned)blocks), dim3(threads), 0, st, y,
                            (long long)m, T(0));
         BHS_HIP(hipGetLastError());
         return BHSPARSE_SUCCESS;
     }
-    hipLaunchKernelGGL(bhs::partition_kernel, dim3((unsigned)((NP + 1 + threads - 1) / threads)),
-                       dim3(threads), 0, st, row_ptr, m, nnz, P, (int)NP, tile_row);
-    BHS_HIP(hipGetLastError());
-    bhs::SegsumParams<T> q;
+    void *base[2] = {nullptr, nullptr};
+    if (int rc = scratch_ptr(base)) return rc;
+    bhs::SegsumParams<T> q{};
     q.m = m;
     q.nnz = nnz;
     q.NP = (int)NP;
     q.TPW = TPW;
     q.NW = (int)NW;
-    q.lead_empty = -1;                                // read from tile_row[0] on the device
-    q.wpb = WPB;
-    q.wave_lds_bytes = (256 + 64 * S * (int)sizeof(T) + 15) / 16 * 16;
+    q.lead_empty = -1;                                // found on the device
     q.alpha = alpha;
-    q.x_lines = 0;
-    hipLaunchKernelGGL((bhs::segsum_kernel<T, S, false, 2, true>),
-                       dim3((unsigned)((NW + WPB - 1) / WPB)), dim3(64 * WPB),
-                       (size_t)WPB * q.wave_lds_bytes, st, row_ptr, col, val, x, y,
-                       (const int *)tile_row, sync_row, sync_val,
-                       (unsigned long long *)nullptr, q);
-    BHS_HIP(hipGetLastError());
-    if (NW > 1) {
-        hipLaunchKernelGGL(bhs::calibrate_kernel<T>, dim3((unsigned)((NW + threads - 1) / threads)),
-                           dim3(threads), 0, st, (const int *)sync_row, (const T *)sync_val,
-                           (int)NW, y);
+    q.x_far = (unsigned long long)n * sizeof(T) > 0xffffffffull;
+    const dim3 grid((unsigned)((NP + WPB - 1) / WPB)), block(64 * WPB);
+    const size_t lds = tile_lds_bytes<T>(S, WPB);
+    if (NW <= kChainWaves) {
+        unsigned call;
+        do call = ++g_noalloc_call & 0x7fffffffu;
+        while (call == 0);
+        hipLaunchKernelGGL((bhs::segsum_tiles_kernel<T, S, 2, true, true, true>), grid, block, lds,
+                           st, row_ptr, col, val, x, y, (const int *)nullptr, (int *)nullptr,
+                           (T *)nullptr,
+                           chain_buf(static_cast<unsigned char *>(base[1]), kChainWaves, call), q);
         BHS_HIP(hipGetLastError());
+        return BHSPARSE_SUCCESS;
     }
+    unsigned char *sb = static_cast<unsigned char *>(base[0]);
+    int *tile_row = reinterpret_cast<int *>(sb);
+    int *sync_row = reinterpret_cast<int *>(sb + o_sr);
+    T *sync_val = reinterpret_cast<T *>(sb + o_sv);
+    hipLaunchKernelGGL(bhs::partition_kernel, dim3((unsigned)((NP + 1 + threads - 1) / threads)),
+                       dim3(threads), 0, st, row_ptr, m, nnz, P, (int)NP, tile_row);
+    BHS_HIP(hipGetLastError());
+    hipLaunchKernelGGL((bhs::segsum_tiles_kernel<T, S, 2, true, false, false>), grid, block, lds,
+                       st, row_ptr, col, val, x, y, (const int *)tile_row, sync_row, sync_val,
+                       bhs::ChainBuf{}, q);
+    BHS_HIP(hipGetLastError());
+    hipLaunchKernelGGL(bhs::calibrate_kernel<T>, dim3((unsigned)((NW + threads - 1) / threads)),
+                       dim3(threads), 0, st, (const int *)sync_row, (const T *)sync_val, (int)NW,
+                       y);
+    BHS_HIP(hipGetLastError());
     return BHSPARSE_SUCCESS;
 }
 

@@ -47,6 +47,7 @@ struct SegsumParams {
     int m, nnz, NP, TPW, NW, lead_empty, wpb, wave_lds_bytes;
     T alpha;
     long long x_lines;   // > 0: x is read ahead into each XCD's L2 (x_lines 128-byte lines)
+    int x_far;           // x reaches past 4 GB (64-bit gather addresses)
 };
 
 // One tile's column indices and values in registers.  Loads are coalesced:
@@ -404,15 +405,13 @@ struct RhsTag {
     static constexpr int value = R;
 };
 
-// BOUNDED: col/val hold exactly nnz items (no padding), so a tile reaching
-// past nnz is loaded with checked indices (a wave-uniform branch).
 // XCH > 0 (fp64, S = 4, KMAX > 1): right-hand-side pairs take their x values
 // from the tile staged in LDS, XCH chunks per item at a time (XStage), at
 // s_stage: 1 KB of column indices, then the staging buffer.
 // NOEMPTY: the matrix has no empty rows (the stacked matrix of the column-panel
 // layout), so no tile is dirty and the empty-row paths are left out.
-template <typename T, int S, int KMAX, bool STRIDED, bool STATS, int CP, bool BOUNDED = false,
-          int XCH = 0, bool NOEMPTY = false>
+template <typename T, int S, int KMAX, bool STRIDED, bool STATS, int CP, int XCH = 0,
+          bool NOEMPTY = false>
 __device__ __forceinline__ void segsum_wave(const MatView<T> &mv, const int w, const int lane,
                                             unsigned *s_head, T *s_buf, T *s_carry, const T alpha,
                                             unsigned long long *stats,
@@ -491,8 +490,7 @@ __device__ __forceinline__ void segsum_wave(const MatView<T> &mv, const int w, c
     // with it (fp32 0.6 us faster, the plain and banded tiles alike).
     constexpr bool kPrefetch = KMAX > 1 || sizeof(T) < 8;
     Tile<T, S> cur;
-    if (BOUNDED && E0 + P > mv.nnz) tile_load_checked<T, S>(mv.col, mv.val, E0, lane, mv.nnz, cur);
-    else tile_load<T, S>(mv.col, mv.val, E0, lane, cur);
+    tile_load<T, S>(mv.col, mv.val, E0, lane, cur);
     constexpr int CR = CP * kWave;              // rows a chunk covers
     RowChunk<CP> rc = load_chunk<CP>(row_ptr, r_first, lane, mv.m);
     int r1 = r_first;
@@ -506,10 +504,7 @@ __device__ __forceinline__ void segsum_wave(const MatView<T> &mv, const int w, c
         r1 = tile_row[p + 1];
         const bool general = r0 != r1;
         if constexpr (!kPrefetch) {
-            if (p != p_begin) {
-                if (BOUNDED && B + P > mv.nnz) tile_load_checked<T, S>(mv.col, mv.val, B, lane, mv.nnz, cur);
-                else tile_load<T, S>(mv.col, mv.val, B, lane, cur);
-            }
+            if (p != p_begin) tile_load<T, S>(mv.col, mv.val, B, lane, cur);
         }
         RhsX<T, S, KMAX> xr;
         [[maybe_unused]] RhsPair<T, S> xp;
@@ -530,11 +525,8 @@ __device__ __forceinline__ void segsum_wave(const MatView<T> &mv, const int w, c
         if (p + 1 < p_end) rc = load_chunk<CP>(row_ptr, r1, lane, mv.m);
         __builtin_amdgcn_sched_barrier(0);
         [[maybe_unused]] Tile<T, S> nxt;
-        if (kPrefetch && p + 1 < p_end) {         // wave-uniform; the last tile loads nothing more
-            const int Bn = B + P;
-            if (BOUNDED && Bn + P > mv.nnz) tile_load_checked<T, S>(mv.col, mv.val, Bn, lane, mv.nnz, nxt);
-            else tile_load<T, S>(mv.col, mv.val, Bn, lane, nxt);
-        }
+        if (kPrefetch && p + 1 < p_end)           // wave-uniform; the last tile loads nothing more
+            tile_load<T, S>(mv.col, mv.val, B + P, lane, nxt);
 
         const bool cont = read_lane(cc.a[0], 0) < B;   // item 0 continues row r0 (lane 0 holds row r0)
         if (p == p_begin) syncing = cont;
@@ -849,9 +841,7 @@ __device__ __forceinline__ void segsum_wave(const MatView<T> &mv, const int w, c
     }
 }
 
-// q.lead_empty < 0: read the number of leading empty rows from tile_row[0]
-// (the first tile's row), for launches that have not copied it to the host.
-template <typename T, int S, bool STATS, int CP, bool BOUNDED = false, bool NOEMPTY = false>
+template <typename T, int S, bool STATS, int CP, bool NOEMPTY = false>
 __global__ __launch_bounds__(512) void segsum_kernel(
     const int *__restrict__ row_ptr, const int *__restrict__ col, const T *__restrict__ val,
     const T *__restrict__ x, T *__restrict__ y, const int *__restrict__ tile_row,
@@ -873,12 +863,595 @@ __global__ __launch_bounds__(512) void segsum_kernel(
     const int w = blk * q.wpb + wib;
     if (w >= q.NW) return;
     unsigned char *wave_lds = reinterpret_cast<unsigned char *>(smem_raw) + wib * q.wave_lds_bytes;
-    const int lead_empty = q.lead_empty >= 0 ? q.lead_empty : tile_row[0];
     MatView<T> mv{row_ptr, tile_row, col, val, x, y, sync_row, sync_val,
-                  q.m, q.nnz, q.NP, q.NW, lead_empty, 1, 1, q.TPW, 0};
-    segsum_wave<T, S, 1, false, STATS, CP, BOUNDED, 0, NOEMPTY>(mv, w, lane, reinterpret_cast<unsigned *>(wave_lds),
-                                       reinterpret_cast<T *>(wave_lds + 256), nullptr, q.alpha,
-                                       stats, nullptr, touch);
+                  q.m, q.nnz, q.NP, q.NW, q.lead_empty, 1, 1, q.TPW, 0};
+    segsum_wave<T, S, 1, false, STATS, CP, 0, NOEMPTY>(
+        mv, w, lane, reinterpret_cast<unsigned *>(wave_lds),
+        reinterpret_cast<T *>(wave_lds + 256), nullptr, q.alpha, stats, nullptr, touch);
+}
+
+// ---------------------------------------------------------------------------
+// One wave per tile: the sums of segsum_wave, bit for bit, with the TPW tiles
+// of a logical wave spread over TPW neighbouring waves of one block.
+//
+// The tile loop runs a logical wave's tiles one after the other because the
+// open row's partial passes from each to the next.  But only the first segment
+// of a tile needs that partial, so here every wave loads, multiplies and reduces
+// its own tile at once, leaves its closing sum in LDS, and after one barrier
+// takes the partial from the tiles before it and redoes that one segment, in the
+// order of the loop.  A matrix of few logical waves then has TPW times as many
+// waves to hide its loads behind (65,536 uniform rows at the default tile, 513
+// logical waves: 14.0 -> 8.2 us in the kernel; 8,000 nonzeros: 10.0 -> 5.5).
+//
+// On large matrices the loop's registers (100 in fp64 at S = 8: 4 waves per
+// SIMD, 58 here: 8) were not the bound, its instructions and LDS conflicts were
+// part of it: SQ counters on the 3x3-block matrix (fp32, 54M nonzeros) put the
+// vector ALU at 47%, the LDS at 37% (two thirds of it bank conflicts of the
+// product transpose) and the texture units at 87% of the time.  So products go
+// to LDS swizzled (swizzle_term: no conflicts left), the lane-sequential
+// reduction has one masked LDS store per item and no other branch, the scan
+// takes its lane conditions from scalar masks, and gathers use 32-bit offsets.
+// Default tile, call with caches warm, fp64: 7-point Laplacian 160^3 91 -> 80 us,
+// 3x3 blocks 160 -> 154, power law (whose gathers miss L2) 119 -> 114.
+// What is left there is memory: 424 MB in 78 us is 5.4 TB/s.  Tried on top and
+// slower: G neighbouring x values per lane in one wide load where columns run on
+// (3x3 blocks fp64 153 -> 170 us: the unit's time is the lines, not the
+// accesses); consecutive items on consecutive lanes (Laplacian fp32 58 -> 62);
+// fewer waves per CU through more LDS (Laplacian 82 -> 90).
+// ---------------------------------------------------------------------------
+constexpr int kMaxGroup = 8;   // waves of a block, and the largest tiles_per_wave
+
+// What the waves of a block hand to each other: every tile's closing sum and
+// its kind (bit 0: inside one row, bit 1: its first item continues a row).
+template <typename T>
+struct TileShare {
+    T val[kMaxGroup];
+    int kind[kMaxGroup];
+};
+
+// Place of 16-byte unit u in a tile's LDS product buffer (U units per lane).
+// A write has consecutive lanes at consecutive units, a read has lane l at unit
+// l*U + j; XORing the low bits with higher ones spreads both over the banks (any
+// 8 or 16 neighbouring lanes hit different 16-byte bank groups).
+template <int U>
+__device__ __forceinline__ int swizzle_term(int u)
+{
+    constexpr int b = U == 1 ? 0 : U == 2 ? 1 : U == 4 ? 2 : 3;
+    return ((u >> 3) ^ (u >> (3 + b))) & (U - 1);
+}
+
+// Segmented inclusive scan of wave_segscan (same sums) on scalar masks: whether
+// a lane adds at a step is its bit of a wave-uniform mask, used as the select's
+// condition directly.
+template <typename T>
+__device__ __forceinline__ T wave_segscan_masked(T v, uint64_t head, int lane)
+{
+    uint64_t cov = head;
+    const int la = lane * 4;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        if (cov == ~0ull) break;
+        T up;
+        if (d == 1) {
+            up = dpp<kDppWaveShr1>(v);
+        } else if constexpr (sizeof(T) == 8) {
+            union { T t; int i[2]; } a, b;
+            a.t = v;
+            b.i[0] = __builtin_amdgcn_ds_bpermute(la + 256 - 4 * d, a.i[0]);
+            b.i[1] = __builtin_amdgcn_ds_bpermute(la + 256 - 4 * d, a.i[1]);
+            up = b.t;
+        } else {
+            up = __int_as_float(__builtin_amdgcn_ds_bpermute(la + 256 - 4 * d, __float_as_int(v)));
+        }
+        const T sum = up + v;
+        v = __builtin_amdgcn_inverse_ballot_w64(cov) ? v : sum;
+        cov |= cov << d;
+    }
+    return v;
+}
+
+__device__ __forceinline__ double zero_where(double v, int mask)
+{
+    union { double d; int i[2]; } u;
+    u.d = v;
+    u.i[0] &= ~mask;
+    u.i[1] &= ~mask;
+    return u.d;
+}
+
+__device__ __forceinline__ float zero_where(float v, int mask)
+{
+    return __int_as_float(__float_as_int(v) & ~mask);
+}
+
+// Rows that cross logical waves, finished inside the launch.  The waves
+// first..last holding one row's nonzeros each send a partial; whoever comes
+// last adds them up, in the order of calibrate_window (wave order within
+// windows of 64 waves, then the first wave's own partial), and stores y.
+// Nobody waits for a wave that has not run.  Words are tagged with the call's
+// number, so that anything another call left behind reads as empty, and are set
+// back to 0 by the wave that finishes the row, so that a replay of the same
+// call starts empty too.  They are written through to, and read from, the
+// point where the eight L2s meet (agent scope).
+struct ChainBuf {
+    unsigned long long *pair;    // [NW * sizeof(T)/4] rows of two waves, by first wave
+    unsigned long long *count;   // [NW] longer rows: tag << 32 | arrivals, by first wave
+    void *own, *part;            // [NW] T: longer rows, the first wave's partial and the others'
+    unsigned call;               // the call's number, 1 .. 2^31 - 1
+};
+
+template <typename U>
+__device__ __forceinline__ U agent_load(const U *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename U>
+__device__ __forceinline__ void agent_store(U *p, U v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Wave w's partial v of `row`, whose nonzeros lie in waves first..last > first.
+template <typename T>
+__device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first, int last, int w,
+                                          T v, int lane, T *__restrict__ y)
+{
+    constexpr int H = sizeof(T) / 4;             // 32-bit halves of a partial
+    const int e0 = first + 1, base = e0 & ~(kWave - 1);
+    const int end = min(last - base, kWave - 1);
+    if (last == e0) {
+        // Two waves swap: lane h exchanges {tag, half h} for what lies there.
+        // The one that finds the other's first half finishes the row; if its
+        // other half is still on its way (it was swapped in the other order),
+        // it replaces this wave's own word shortly.
+        const unsigned tag = cb.call << 1 | (w == first ? 0u : 1u);   // the two sides differ
+        unsigned half;
+        if constexpr (H == 2) {
+            const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+            half = (unsigned)(lane == 0 ? b : b >> 32);
+        } else {
+            half = __builtin_bit_cast(unsigned, v);
+        }
+        unsigned long long *p = cb.pair + (long long)first * H + lane;
+        unsigned long long got = 0ull;
+        if (lane < H)
+            got = __hip_atomic_exchange(p, (unsigned long long)tag << 32 | half, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned other = tag ^ 1u;
+        if (__builtin_amdgcn_readfirstlane((unsigned)(got >> 32)) != other) return;
+        if (lane < H) {
+            for (int i = 0; i < (1 << 16) && (unsigned)(got >> 32) != other; ++i) got = agent_load(p);
+            agent_store(p, 0ull);
+        }
+        const unsigned lo = (unsigned)read_lane((int)(unsigned)got, 0);
+        T o;
+        if constexpr (H == 2) {
+            const unsigned hi = (unsigned)read_lane((int)(unsigned)got, 1);
+            o = __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+        } else {
+            o = __builtin_bit_cast(float, lo);
+        }
+        const T head = w == first ? v : o;
+        T tot = w == first ? o : v;
+        if (end == kWave - 1) tot = tot + T(0);       // as at a window's last entry
+        if (lane == 0) y[row] = head + tot;
+        return;
+    }
+    T *own = reinterpret_cast<T *>(cb.own), *part = reinterpret_cast<T *>(cb.part);
+    const unsigned others = (unsigned)(last - first);
+    int complete = 0;
+    if (lane == 0) {
+        agent_store(w == first ? own + first : part + w, v);
+        // the partial has arrived before the count says so
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const unsigned long long tag = (unsigned long long)cb.call << 32;
+        unsigned long long seen = 0ull;
+        // the first to arrive sets the tag; the rest add to it
+        while (seen >> 32 != cb.call)
+            if (__hip_atomic_compare_exchange_strong(cb.count + first, &seen, tag | 1ull,
+                                                     __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT))
+                break;
+        if (seen >> 32 == cb.call)
+            complete = (unsigned)__hip_atomic_fetch_add(cb.count + first, 1ull, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT) == others;
+        asm volatile("" ::: "memory");
+    }
+    if (!__builtin_amdgcn_readfirstlane(complete)) return;
+    const int e = base + lane;
+    const bool on = e >= e0 && e <= last;
+    const T pv = on ? agent_load(part + e) : T(0);
+    T tot = read_lane(wave_segscan(pv, 1ull << (e0 - base) | 1ull, lane), end);
+    if (end == kWave - 1) {                 // up to a window's last entry: later windows follow
+        T ext = T(0);
+        for (int nb = base + kWave; nb <= last; nb += kWave) {
+            const T pn = nb + lane <= last ? agent_load(part + nb + lane) : T(0);
+            ext = ext + wave_sum(pn);
+        }
+        tot = tot + ext;
+    }
+    if (lane == 0) {
+        const T head = w == first ? v : agent_load(own + first);
+        y[row] = head + tot;
+        agent_store(cb.count + first, 0ull);
+    }
+}
+
+// The last row r >= lo with row_ptr[r] <= key, given row_ptr[lo] = vlo <= key.
+// A round cuts the bracket into 17 parts (16 probes: 64 would need a round less,
+// but each is a cache line, and the line rate from L2 is what gathers wait for:
+// power law, 10M nonzeros, fp32, 73.6 us a call with 64, 68.4 with 16 or 8), then
+// reads the 256 rows around the place where rows of even length would put key.
+// Between even rows that finds it at once; otherwise the bracket has shrunk.  `guesses`: rounds at the start that read the 256 rows only (two where
+// even_rows says so: a stencil's border rows put the first guess off by some
+// thousand rows, and the second, from the edge of the first, right).
+__device__ __forceinline__ int find_row(const int *__restrict__ row_ptr, int m, int nnz, int key,
+                                        int lo, int vlo, int guesses, int lane)
+{
+    constexpr int W = 4 * kWave, kProbes = 16;
+    int hi = m + 1, vhi = nnz;             // row_ptr[hi] > key (past the end at first)
+    for (;; --guesses) {
+        if (guesses <= 0 && hi - lo > W) {
+            const int i = min(lane, kProbes - 1) + 1;
+            const int at = lo + (int)((long long)(hi - lo) * i / (kProbes + 1));
+            const int v = row_ptr[at];
+            const int n = __popcll(ballot(v <= key && lane < kProbes));   // a prefix of the lanes
+            if (n < kProbes) hi = read_lane(at, n), vhi = read_lane(v, n);
+            if (n > 0) lo = read_lane(at, n - 1), vlo = read_lane(v, n - 1);
+        }
+        int g = lo;
+        if (hi - lo > W) {
+            const float f = (float)(key - vlo) / (float)max(vhi - vlo, 1) * (float)(hi - lo);
+            g = __builtin_amdgcn_readfirstlane(lo + (int)f) - W / 2;
+            g = max(lo, min(g, hi - W));
+        }
+        // rows [g, g + W) of the bracket; the whole bracket if it is no longer
+        int v[4], n = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = row_ptr[min(g + q * kWave + lane, m)];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) n += __popcll(ballot(g + q * kWave + lane < hi && v[q] <= key));
+        if (hi - lo <= W || (n > 0 && n < W)) return g + n - 1;
+        if (n == 0) hi = g, vhi = read_lane(v[0], 0);
+        else lo = g + W - 1, vlo = read_lane(v[3], kWave - 1);
+    }
+}
+
+// Whether the middle row starts within 128 rows of where rows of even length
+// would put it (bands, stencils, dense blocks; hardly ever a power law).
+__device__ __forceinline__ bool even_rows(const int *__restrict__ row_ptr, int m, int nnz)
+{
+    const int h = m >> 1;
+    const float per = (float)nnz / (float)m;
+    return fabsf((float)row_ptr[h] - per * (float)h) < 128.0f * per;
+}
+
+// BOUNDED: col/val hold exactly nnz items (no padding), so a tile reaching
+// past nnz is loaded with checked indices (a wave-uniform branch).  SEARCH: no
+// tile_row; each wave finds its first row (while its stream is on its way) and
+// its last from the row chunk.  FUSED: rows crossing logical waves are finished
+// here (chain_add), else their partials are left to calibrate_kernel.
+template <typename T, int S, int CP, bool BOUNDED, bool SEARCH, bool FUSED>
+__global__ __launch_bounds__(512) void segsum_tiles_kernel(
+    const int *__restrict__ row_ptr, const int *__restrict__ col, const T *__restrict__ val,
+    const T *__restrict__ x, T *__restrict__ y, const int *__restrict__ tile_row,
+    int *__restrict__ sync_row, T *__restrict__ sync_val, const ChainBuf cb,
+    const SegsumParams<T> q)
+{
+    constexpr int P = kWave * S;
+    constexpr int G = Tile<T, S>::G, U = S / G;
+    constexpr int CR = CP * kWave;
+    typedef T unit_t __attribute__((ext_vector_type(G)));
+    extern __shared__ double smem_raw[];
+    const int lane = lane_id();
+    int touch = 0;
+    {
+        const long long t = (long long)(blockIdx.x / 8) * blockDim.x + threadIdx.x;
+        if (t < q.x_lines) touch = reinterpret_cast<const int *>(x)[t * (128 / sizeof(int))];
+    }
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nwb = blockDim.x >> 6;
+    const int p = xcd_remap((int)blockIdx.x, (int)gridDim.x) * nwb + wib;
+    const int TPW = q.TPW;                      // a power of two
+    const int g0 = wib & ~(TPW - 1);            // the logical wave's first tile in the block
+    const int w = p >> __builtin_ctz(TPW);
+    // product buffers first (16-byte aligned), then the head words, then the hand-over
+    unit_t *su = reinterpret_cast<unit_t *>(smem_raw) + wib * (kWave * U);
+    T *sb = reinterpret_cast<T *>(su);
+    unsigned *s_head = reinterpret_cast<unsigned *>(reinterpret_cast<T *>(smem_raw) + nwb * P) +
+                       wib * kWave;
+    TileShare<T> &sh = *reinterpret_cast<TileShare<T> *>(
+        reinterpret_cast<unsigned *>(reinterpret_cast<T *>(smem_raw) + nwb * P) + nwb * kWave);
+    const bool active = p < q.NP;
+    const int pe = active ? p : 0;
+    const int B = pe * P;
+    const T alpha = q.alpha;
+
+    Tile<T, S> t;
+    if (BOUNDED && B + P > q.nnz) tile_load_checked<T, S>(col, val, B, lane, q.nnz, t);
+    else tile_load<T, S>(col, val, B, lane, t);
+    int r0, r1;
+    if constexpr (SEARCH) {
+        const int guesses = even_rows(row_ptr, q.m, q.nnz) ? 2 : 0;
+        r0 = find_row(row_ptr, q.m, q.nnz, B, 0, 0, guesses, lane);
+    } else {
+        r0 = tile_row[pe];
+        r1 = active ? tile_row[pe + 1] : r0;
+    }
+    const RowChunk<CP> cc = load_chunk<CP>(row_ptr, r0, lane, q.m);
+    __builtin_amdgcn_sched_barrier(0);
+    T prod[S];
+    {
+        T xv[S];
+        if (q.x_far) {
+#pragma unroll
+            for (int k = 0; k < S; ++k) xv[k] = x[t.c[k]];
+        } else {                      // x below 4 GB: 32-bit offsets, one instruction each
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                xv[k] = *reinterpret_cast<const T *>(reinterpret_cast<const char *>(x) +
+                                                     (unsigned)t.c[k] * (unsigned)sizeof(T));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::"v"(touch));   // emits no instruction
+#pragma unroll
+        for (int k = 0; k < S; ++k) prod[k] = t.v[k] * xv[k];
+        if (B + P > q.nnz) {
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                prod[k] = keep_or_zero(prod[k], tile_item<T, S>(B, lane, k) < q.nnz);
+        }
+    }
+    if constexpr (SEARCH) {
+        // the last row starting at or before the tile's end: count the chunk's
+        // starts up to there, and search on only if all of them are
+        r1 = r0;
+        if (active) {
+            const int key = min(B + P, q.nnz);
+            int cnt = 0;
+            static_for<CP>([&](auto qc) {
+                cnt += __popcll(ballot(cc.a[qc] <= key && r0 + qc * kWave + lane <= q.m));
+            });
+            r1 = r0 + cnt - 1;
+            if (cnt == CR)
+                r1 = find_row(row_ptr, q.m, q.nnz, key, r1, read_lane(cc.a[CP - 1], kWave - 1), 0,
+                              lane);
+        }
+    }
+    // rows before the first nonzero belong to no tile: spread their zeroing
+    int lead_empty = q.lead_empty;              // < 0: not known to the host
+    if constexpr (SEARCH)
+        lead_empty = row_ptr[1] > 0 ? 0 : find_row(row_ptr, q.m, q.nnz, 0, 0, 0, 0, lane);
+    else if (lead_empty < 0)
+        lead_empty = tile_row[0];
+    if (lead_empty > 0 && active) {
+        const unsigned per = ((unsigned)lead_empty + (unsigned)q.NP - 1) / (unsigned)q.NP;
+        const long long lo = (long long)p * per;
+        const long long hi = min(lo + per, (long long)lead_empty);
+        for (long long r = lo + lane; r < hi; r += kWave) y[r] = T(0);
+    }
+
+    const bool general = r0 != r1;
+    const int rp_r1 = row_ptr[min(r1, q.m)], rp_next = row_ptr[min(r1 + 1, q.m)];
+    const bool cont = read_lane(cc.a[0], 0) < B;   // item 0 continues row r0
+    const int stop = (r1 == q.m) ? q.m - 1 : r1;
+    const bool big = r1 - r0 >= CR;
+    uint64_t mne[CP];
+    unsigned hb = 0;
+    bool dirty = false, partial_tail = false;
+    int seg_base = 0, K = 0;
+    T acc = T(0), I = T(0), out_val;
+    T pc[S];
+    uint64_t present = 1;
+    if (general) {
+        // ---- bit flags
+        bool lane_dirty = false;
+        s_head[lane] = 0u;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {                  // products in tile order
+            unit_t u;
+#pragma unroll
+            for (int g = 0; g < G; ++g) u[g] = prod[j * G + g];
+            const int term = swizzle_term<U>(lane) ^ swizzle_term<U>(j * kWave);
+            su[j * kWave + (lane ^ term)] = u;
+        }
+        wave_sync();
+        static_for<CP>([&](auto qc) {
+            constexpr int qq = decltype(qc)::value;
+            mne[qq] = 0ull;
+            if (qq > 0 && r0 + qq * kWave > stop) return;   // wave-uniform: no rows here
+            const bool have = r0 + qq * kWave + lane <= stop;
+            const bool ne = have && chunk_next<qq>(cc, lane) > cc.a[qq];
+            lane_dirty = lane_dirty || (have && !ne);
+            mne[qq] = ballot(ne);
+            const unsigned o = (unsigned)(cc.a[qq] - B);
+            if (ne && o < (unsigned)P) atomicOr(&s_head[o / S], 1u << (o % S));
+        });
+        if (big)
+            for (int rb = r0 + CR; rb <= stop;) {          // >= CR rows
+                const int rq = min(rb + lane, stop);
+                const int rp = row_ptr[rq];
+                const unsigned o = (unsigned)(rp - B);
+                const int rpn = row_ptr[rq + 1];
+                const int vb = row_ptr[min(rb + kWave, stop + 1)];
+                if (rb + kWave <= stop && read_lane(rp, 0) == vb) {
+                    // 64 empty rows with more rows after them: skip the whole run
+                    const int re = empty_run_end(row_ptr, rb + kWave, vb, stop);
+                    lane_dirty = true;
+                    for (int r = rb + lane; r < re; r += kWave) y[r] = T(0);
+                    rb = re;
+                    continue;
+                }
+                if (rb + lane <= stop) {
+                    if (rpn > rp) {
+                        if (o < (unsigned)P) atomicOr(&s_head[o / S], 1u << (o % S));
+                    } else {
+                        lane_dirty = true;
+                        y[rb + lane] = T(0);
+                    }
+                }
+                rb += kWave;
+            }
+        dirty = ballot(lane_dirty) != 0ull;
+        wave_sync();
+        hb = s_head[lane];
+        if (lane == 0) hb |= 1u;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const unit_t u = su[lane * U + (j ^ swizzle_term<U>(lane * U))];
+#pragma unroll
+            for (int g = 0; g < G; ++g) pc[j * G + g] = u[g];
+        }
+        wave_sync();
+        // ---- segment numbers
+        const int nh = __popc(hb);
+        const int incl = wave_incl_scan(nh, lane);
+        seg_base = incl - nh;
+        K = read_lane(incl, kWave - 1);
+        partial_tail = (r1 < q.m) && (rp_r1 < B + P);
+        // the tile loop starts a logical wave with a carry of +0
+        if (lane == 0 && cont && wib == g0) pc[0] = pc[0] + T(0);
+        // ---- lane-sequential segmented reduction: every head closes the sum
+        // before it, the lane's first one for the segment of the lanes before
+        int sidx = lane == 0 ? -1 : seg_base - 1;
+#pragma unroll
+        for (int kk = 0; kk < S; ++kk) {
+            const int h = __builtin_amdgcn_sbfe((int)hb, kk, 1);   // -1 at a head
+            if (kk == 0) {
+                if (h && lane > 0) sb[sidx] = T(0);
+            } else if (h) {
+                sb[sidx] = acc;
+            }
+            sidx -= h;
+            acc = zero_where(acc, h);
+            acc += pc[kk];
+        }
+        present = ballot(hb != 0u);
+        I = wave_segscan_masked(acc, present, lane);
+        out_val = read_lane(I, kWave - 1);
+    } else {
+        T s = prod[0];
+#pragma unroll
+        for (int k = 1; k < S; ++k) s += prod[k];
+        s = wave_sum(s);
+        out_val = (cont && wib == g0) ? T(0) + s : s;
+    }
+
+    bool lead_open = cont;       // the row open at the logical wave's start still is
+    bool need = false;
+    T carry = T(0);
+    if (TPW > 1) {
+        if (lane == 0) {
+            sh.val[wib] = out_val;
+            sh.kind[wib] = (general ? 0 : 1) | (cont ? 2 : 0);
+        }
+        __syncthreads();
+        if (!active) return;
+        if (wib > g0) {
+            need = cont;
+            const int kd = sh.kind[lane & (kMaxGroup - 1)];
+            const unsigned fast = (unsigned)ballot(lane < kMaxGroup && (kd & 1));
+            const unsigned conts = (unsigned)ballot(lane < kMaxGroup && (kd & 2));
+            const unsigned below = ((1u << wib) - 1) & ~((1u << g0) - 1);   // its earlier tiles
+            // the nearest earlier tile whose closing sum needs no carry
+            const unsigned stops = below & ~(fast & conts);
+            const int j = stops ? 31 - __builtin_clz(stops) : g0;
+            carry = sh.val[j];
+            for (int jj = j + 1; jj < wib; ++jj) carry = carry + sh.val[jj];
+            lead_open = ((conts >> g0) & 1u) && (below & ~fast) == 0;
+        }
+    } else if (!active) {
+        return;
+    }
+    const bool last = p == min((w + 1) * TPW, q.NP) - 1;
+    [[maybe_unused]] const int wsh = __builtin_ctz(TPW * P);      // nonzero -> logical wave
+    [[maybe_unused]] int sync_key = -1;
+    [[maybe_unused]] T sync_v = T(0);
+    if (general) {
+        if (need) {
+            // the carry starts lane 0's first sum: only the first segment changes
+            T a0 = pc[0] + carry;
+            unsigned hl = hb & ~1u;
+#pragma unroll
+            for (int kk = 1; kk < S; ++kk) {
+                const T n = a0 + pc[kk];
+                if (!(hl & ((2u << kk) - 1))) a0 = n;
+            }
+            if (lane == 0) {
+                if (hl) sb[0] = a0;
+                else acc = a0;
+            }
+            I = wave_segscan_masked(acc, present, lane);
+        }
+        const T Iprev = dpp<kDppWaveShr1>(I);
+        if (hb && lane > 0) sb[seg_base - 1] = Iprev + sb[seg_base - 1];
+        if (lane == kWave - 1) sb[K - 1] = I;
+        wave_sync();
+        const int kb = lead_open ? 1 : 0;
+        const int ke = partial_tail ? K - 1 : K;
+        if (!dirty) {
+            for (int kk = kb + lane; kk < ke; kk += kWave) y[(long long)r0 + kk] = alpha * sb[kk];
+        } else {
+            int running = 0;
+            static_for<CP>([&](auto qc) {
+                constexpr int qq = decltype(qc)::value;
+                if (qq > 0 && r0 + qq * kWave > stop) return;
+                const int row = r0 + qq * kWave + lane;
+                const bool ne = __builtin_amdgcn_inverse_ballot_w64(mne[qq]);
+                const int rank = running + popc_below(mne[qq]);
+                if (ne && rank >= kb && rank < ke) y[row] = alpha * sb[rank];
+                else if (row <= stop && !ne) y[row] = T(0);
+                running += __popcll(mne[qq]);
+            });
+            if (big)
+                for (int rb = r0 + CR; rb <= stop;) {
+                    const int rq = min(rb + lane, stop);
+                    const int rp = row_ptr[rq], rpn = row_ptr[rq + 1];
+                    const int vb = row_ptr[min(rb + kWave, stop + 1)];
+                    if (rb + kWave <= stop && read_lane(rp, 0) == vb) {
+                        rb = empty_run_end(row_ptr, rb + kWave, vb, stop);   // no segments
+                        continue;
+                    }
+                    const int r = rb + lane;
+                    const bool ne = r <= stop && rpn > rp;
+                    const uint64_t msk = ballot(ne);
+                    const int rank = running + popc_below(msk);
+                    if (ne && rank >= kb && rank < ke) y[r] = alpha * sb[rank];
+                    running += __popcll(msk);
+                    rb += kWave;
+                }
+        }
+        if (lead_open) {     // the row began in an earlier logical wave and ends here
+            if constexpr (FUSED)
+                chain_add(cb, r0, read_lane(cc.a[0], 0) >> wsh, w, w, alpha * sb[0], lane, y);
+            sync_key = r0;
+            sync_v = alpha * sb[0];
+        }
+        if (last && partial_tail) {
+            if constexpr (FUSED)
+                chain_add(cb, r1, w, (rp_next - 1) >> wsh, w, alpha * sb[K - 1], lane, y);
+            else if (lane == 0) y[r1] = alpha * sb[K - 1];
+        }
+    } else if (last) {
+        const T tot = alpha * (need ? carry + out_val : out_val);
+        if constexpr (FUSED) {
+            const int first = lead_open ? read_lane(cc.a[0], 0) >> wsh : w;
+            chain_add(cb, r1, first, (rp_next - 1) >> wsh, w, tot, lane, y);
+        } else if (lead_open) {
+            sync_key = r1;
+            sync_v = tot;
+        } else if (lane == 0) {
+            y[r1] = tot;
+        }
+    }
+    if constexpr (!FUSED) {
+        // the wave that closes (or passes on) a row from an earlier logical
+        // wave leaves its partial to calibrate_kernel; none: -1
+        if (lane == 0 && (sync_key >= 0 || (wib == g0 && !cont))) {
+            sync_row[w] = sync_key;
+            if (sync_key >= 0) sync_val[w] = sync_v;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1034,7 +1607,7 @@ __global__ __launch_bounds__(512) void batched_kernel(
                       sync_row + md.sync_off, sync_val + (long long)md.sync_off * KMAX,
                       md.m, md.nnz, md.NP, md.NW, md.lead_empty, md.k, md.k, TPW,
                       (int)md.y_off};
-        segsum_wave<T, S, KMAX, true, false, 2, false, XCH>(mv, iw.y, lane, s_head, s_buf,
+        segsum_wave<T, S, KMAX, true, false, 2, XCH>(mv, iw.y, lane, s_head, s_buf,
                                                            s_carry, alpha, nullptr, s_stage);
         if (lane == 0) sync_k[md.sync_off + iw.y] = md.k;
         wave_sync();                              // LDS is reused by the next item

@@ -259,15 +259,16 @@ int bhs_d_apply_tuner_topk(bhs_handle_t h, bhs_mlp_t net, const bhs_config *clas
  * forbid hipMalloc): y = alpha * A * x over the caller's DEVICE arrays
  * (row_ptr[m+1], col[nnz], val[nnz], x[n], y[m]; col and val 16-byte
  * aligned), enqueued on `stream` (a hipStream_t, NULL = the null stream) and
- * not waited for.  It runs the kernels of a handle's default tile (segmented
- * sum, 8 items per lane, 4 waves per block, 4 tiles per wave, plain layout),
- * so y equals bhs_*_spmv's with that tile bit for bit, with the tile
- * partition and the cross-wave partials in a static device scratch array of
- * 8 MiB per device (held until the process ends).  It calls no hipMalloc,
- * hipFree, memset or copy.  A matrix needing more scratch than that
- * ((nnz/512 + 1) * 4 bytes of partition plus (nnz/2048) * (4 + sizeof(T))
- * bytes of partials, about 600M nonzeros in fp64) is refused with
- * BHSPARSE_INVALID_ARGUMENT.  The caller guarantees a valid CSR (row_ptr
+ * not waited for.  It computes the sums of a handle's default tile (segmented
+ * sum, 8 items per lane, 4 waves per block, 4 tiles per wave, plain layout), so
+ * y equals bhs_*_spmv's with that tile bit for bit, in one kernel launch up to
+ * 134M nonzeros and three beyond (partition, segmented sum, calibration).  The
+ * partials of rows that cross waves and, beyond 134M nonzeros, the partition
+ * sit in static device arrays of 10.5 MiB per device (held until the process
+ * ends).  It calls no hipMalloc, hipFree, memset or copy.  A matrix needing more
+ * than 8 MiB for ((nnz/512 + 1) * 4 bytes of partition plus (nnz/2048) *
+ * (4 + sizeof(T)) bytes of partials, about 600M nonzeros in fp64) is refused
+ * with BHSPARSE_INVALID_ARGUMENT.  The caller guarantees a valid CSR (row_ptr
  * monotone from 0 to nnz, 0 <= col < n): device data is not checked.
  * Every call on a device shares its scratch: calls that overlap on one device
  * (two host threads, or two streams) race and must be serialised. */

@@ -1,0 +1,176 @@
+"""The one-wave-per-tile kernel against the lane-exact model and the tile loop
+(GPU): y must be the same bits for every tile shape it is built for, with the
+rows that cross logical waves finished inside the launch, and with the rows
+found inside it (the allocation-free entry point)."""
+import numpy as np
+import pytest
+
+import cases
+import kernel_model as km
+from benchmark_spmv_using_csr_amd import _lib, matgen
+from benchmark_spmv_using_csr_amd.spmv import bhsparse_spmv
+from test_zz_no_alloc import DeviceArrays, call_noalloc
+
+pytestmark = pytest.mark.gpu
+
+
+def lengths_around(P, T, waves, seed):
+    """Row lengths over `waves` logical waves of T tiles of P nonzeros that meet
+    tile and wave ends every way: rows ending on them and one to either side,
+    rows inside a tile, over a tile, over two and many logical waves, runs of
+    empty rows across the ends; empty rows first and last."""
+    rng = np.random.default_rng(seed)
+    lens, at = [0] * 7, 0
+    total = waves * P * T + 13
+
+    def add(n):
+        nonlocal at
+        lens.append(int(n))
+        at += int(n)
+
+    kind = 0
+    while at < total:
+        kind += 1
+        to_tile, to_wave = P - at % P, P * T - at % (P * T)
+        pick = kind % 9
+        if pick == 0:
+            add(to_tile)                        # ends on a tile's end
+        elif pick == 1:
+            add(to_wave)                        # ends on a logical wave's end
+            lens.extend([0] * int(rng.integers(1, 4)))
+        elif pick == 2:
+            add(to_wave + 1)
+        elif pick == 3:
+            add(max(to_wave - 1, 1))
+            add(2)                              # one item on each side of the end
+        elif pick == 4:
+            add(to_wave + P * T)                # the rest of this wave and all of the next
+        elif pick == 5 and kind % 2:
+            add(to_wave + 2 * P * T + 5)        # four waves
+        elif pick == 6:
+            lens.extend([0] * int(rng.choice([3, 70, 150, 300])))
+            add(3)
+        else:
+            for n in rng.integers(1, 40, 30):
+                add(n)
+                if rng.random() < 0.1:
+                    lens.append(0)
+    return lens + [0] * 5
+
+
+@pytest.mark.parametrize("S", [4, 8, 16])
+@pytest.mark.parametrize("T", [1, 2, 4, 8])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_every_shape_against_the_model(S, T, dtype):
+    # over 32 logical waves, so that T > 1 leaves the tile loop too
+    c = cases.from_lengths(f"S={S} T={T}", lengths_around(64 * S, T, 40, 10 * S + T),
+                           n=4 * 64 * S * T + 100, seed=S)
+    c.val = c.val.astype(dtype)
+    c.x = c.x.astype(dtype)
+    assert c.nnz > 33 * 64 * S * T
+    for wpb in (1, 4):
+        op = bhsparse_spmv(dtype)
+        _lib.check(op.init_platform(0), "init_platform")
+        _lib.check(op.set_config(0, S, wpb, T, 0), "set_config")
+        y = np.full(c.m, np.nan, dtype)
+        _lib.check(op.prepare_mem(c.m, c.n, c.nnz, c.row_ptr, c.col, c.val, c.x, y), "prepare_mem")
+        print(f"[gpu] tiles S={S} T={T} wpb={wpb} {np.dtype(dtype).name} nnz={c.nnz}", flush=True)
+        ym = km.segsum(c.row_ptr, c.col, c.val, c.x, S=S, TPW=T, alpha=0.75, dtype=dtype)
+        for _ in range(2):                      # a second call finds its words empty
+            _lib.check(op.spmv(0.75), "spmv")
+            _lib.check(op.get_y(), "get_y")
+            assert np.array_equal(y, ym), np.flatnonzero(y != ym)[:8]
+        op.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_rows_over_many_logical_waves(dtype):
+    """Rows over 3, 63, 64, 65 and 200 logical waves (windows of 64 partials),
+    between short ones."""
+    PW = 64 * 4
+    lens = [5, 3 * PW, 9, 63 * PW + 7, 1, 64 * PW, 2, 65 * PW - 3, 0, 4, 200 * PW + 1, 6]
+    c = cases.from_lengths("long rows", lens, n=201 * PW, seed=3)
+    v, x = c.val.astype(dtype), c.x.astype(dtype)
+    op = bhsparse_spmv(dtype)
+    _lib.check(op.init_platform(0), "init_platform")
+    _lib.check(op.set_config(0, 4, 1, 1, 0), "set_config")
+    y = np.zeros(c.m, dtype)
+    _lib.check(op.prepare_mem(c.m, c.n, c.nnz, c.row_ptr, c.col, v, x, y), "prepare_mem")
+    print(f"[gpu] rows over many waves {np.dtype(dtype).name}", flush=True)
+    ym = km.segsum(c.row_ptr, c.col, v, x, S=4, TPW=1, dtype=dtype)
+    for _ in range(3):
+        _lib.check(op.spmv(1.0), "spmv")
+        _lib.check(op.get_y(), "get_y")
+        assert np.array_equal(y, ym)
+
+
+def row_layouts():
+    rng = np.random.default_rng(8)
+    even = np.full(60_000, 9)
+    skewed = np.concatenate([np.full(40_000, 1), np.full(20_000, 25)])
+    late = np.concatenate([np.zeros(50_000, int), rng.integers(0, 20, 30_000), np.zeros(40_000, int)])
+    pareto = np.minimum((rng.pareto(1.0, 50_000) * 2).astype(int), 30_000)
+    holes = np.tile(np.r_[np.full(300, 8), np.zeros(5000, int)], 20)
+    mirrored = np.concatenate([np.full(9000, 3), np.full(9000, 15), np.full(9000, 15),
+                               np.full(9000, 3)])        # the middle row is where even rows put it
+    return {"even": even, "skewed": skewed, "empty ends": late, "pareto": pareto, "holes": holes,
+            "mirrored": mirrored, "few rows": np.full(255, 300), "257 rows": np.full(257, 300),
+            "one row": np.array([300_000])}
+
+
+@pytest.mark.parametrize("name", list(row_layouts()))
+def test_rows_found_inside_the_launch(name):
+    """Against a handle with the default tile, whose rows partition_kernel finds."""
+    lens = row_layouts()[name]
+    rng = np.random.default_rng(len(lens))
+    m, n, nnz = len(lens), 300_000, int(lens.sum())
+    row_ptr = np.r_[0, np.cumsum(lens)].astype(np.int32)
+    col = rng.integers(0, n, nnz).astype(np.int32)
+    val, x = rng.uniform(-1, 1, nnz), rng.uniform(-1, 1, n)
+    print(f"[gpu] rows found inside the launch: {name} m={m} nnz={nnz}", flush=True)
+    op = bhsparse_spmv(np.float64)
+    _lib.check(op.init_platform(0), "init_platform")
+    y = np.zeros(m)
+    _lib.check(op.prepare_mem(m, n, nnz, row_ptr, col, val, x, y), "prepare_mem")
+    _lib.check(op.spmv(-0.5), "spmv")
+    _lib.check(op.get_y(), "get_y")
+    with DeviceArrays(row_ptr, col, val, x, np.full(m, np.nan)) as d:
+        for _ in range(2):
+            _lib.check(call_noalloc(np.float64, m, n, nnz, d.ptrs, -0.5), "spmv_noalloc")
+            assert np.array_equal(d.get(4, y), y)
+
+
+def test_beyond_the_one_kernel_sizes():
+    """More logical waves than the one-kernel path has words for (134M nonzeros):
+    partition, kernel and calibration; whole numbers, so the sums are exact."""
+    nnz, m, n = 65536 * 2048 + 3001, 1_000_003, 1000
+    row_ptr = (np.arange(m + 1, dtype=np.int64) * nnz // m).astype(np.int32)
+    row_ptr[500_001:500_020] = row_ptr[500_020]                   # a row of 2,700 and empty rows
+    col = np.arange(nnz, dtype=np.int32) % n
+    x = (np.arange(n) % 7 - 3).astype(np.float32)
+    print(f"[gpu] {nnz} nonzeros through spmv_noalloc", flush=True)
+    sums = np.r_[0, np.cumsum(x.astype(np.int64)[col])]
+    y0 = np.full(m, np.nan, np.float32)
+    with DeviceArrays(row_ptr, col, np.ones(nnz, np.float32), x, y0) as d:
+        _lib.check(call_noalloc(np.float32, m, n, nnz, d.ptrs, 1.0), "spmv_noalloc")
+        y = d.get(4, y0)
+    assert np.array_equal(y.astype(np.int64), sums[row_ptr[1:]] - sums[row_ptr[:-1]])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_more_logical_waves_than_the_fused_launch_takes(dtype):
+    """A handle's default tile over 16,384 logical waves (kernel, then
+    calibration) against the allocation-free entry point (one kernel)."""
+    A = matgen.uniform_rows(21, 1_300_000, 900_000, 0, 56)
+    assert A.nnz > 16384 * 2048
+    v, x = A.val.astype(dtype), matgen.vector(22, A.n).astype(dtype)
+    print(f"[gpu] {A.nnz} nonzeros {np.dtype(dtype).name}", flush=True)
+    op = bhsparse_spmv(dtype)
+    _lib.check(op.init_platform(0), "init_platform")
+    y = np.zeros(A.m, dtype)
+    _lib.check(op.prepare_mem(A.m, A.n, A.nnz, A.row_ptr, A.col, v, x, y), "prepare_mem")
+    _lib.check(op.spmv(1.5), "spmv")
+    _lib.check(op.get_y(), "get_y")
+    with DeviceArrays(A.row_ptr, A.col, v, x, np.full(A.m, np.nan, dtype)) as d:
+        _lib.check(call_noalloc(dtype, A.m, A.n, A.nnz, d.ptrs, 1.5), "spmv_noalloc")
+        assert np.array_equal(d.get(4, y), y)
