@@ -551,10 +551,13 @@ size_t tile_lds_bytes(int S, int waves)
 //    (26k) 167 / 164 / 163, warm 160 / 153 / 153.  The fused end of a wave (an
 //    exchange past the L2s) is cheaper than a launch of calibrate_kernel until
 //    the device is full of waves for many rounds: up to 16,384.
-//  * T = 1 is one wave per tile anyway; only the fused end gains: S = 8, 65,536
-//    rows (2k) 13.2 -> 11.8, band of 27 (16k) 29.5 -> 26.8, Laplacian 160^3 (56k)
-//    102 -> 104.  S = 4 has half the work per exchange: 65,536 rows (4.1k) 13.4 ->
-//    12.4, 2M-nonzero power law (7.8k) 22.2 -> 22.7: up to 4,096.
+//  * T = 1 is one wave per tile anyway; only the fused end gains, as long as the
+//    device is not full of waves many times over (loop / fused, warm): S = 8,
+//    2M nonzeros (3.9k), 3x3 blocks fp64 10.7 / 8.6, fp32 9.8 / 8.4, uniform
+//    rows 15.9 / 15.5; 6M (12k), 3x3 blocks fp32 16.4 / 18.1, uniform rows fp64
+//    39.4 / 42.7: up to 4,096.  S = 4 has half the work per exchange; 1M (3.9k):
+//    uniform rows 10.7 / 9.1, band of 41 8.4 / 6.1, power law with one row
+//    over 390 waves 12.3 / 13.3; 2M (7.8k), power law 22.2 / 22.7.
 //  * fp32, S = 4 (2 KB of A a wave), T = 4, Laplacian 160^3: 63.9 / 70.8 warm.
 //  * T > 1 with up to 32 logical waves (65,000 nonzeros at the default tile)
 //    stays on the loop, 14 us against 6: the fixed default tile is the yardstick
@@ -571,7 +574,7 @@ SegsumKernel pick_kernel(const Impl<T> *im, long long NW)
         return kWaveLoop;
     if (tile_lds_bytes<T>(S, tile_block_waves(c)) > im->dev_lds) return kWaveLoop;
     if (TPW > 1 && NW <= 32) return kWaveLoop;
-    if (NW <= (S == 4 ? 4096 : 16384)) return kTilePerWaveFused;
+    if (NW <= (TPW == 1 || S == 4 ? 4096 : 16384)) return kTilePerWaveFused;
     return TPW == 1 || S * sizeof(T) < 32 ? kWaveLoop : kTilePerWave;
 }
 
