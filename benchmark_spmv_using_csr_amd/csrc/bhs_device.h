@@ -155,25 +155,6 @@ __device__ __forceinline__ float2v read_lane(float2v v, int l)
     return float2v{read_lane(v.x, l), read_lane(v.y, l)};
 }
 
-// lane i <- lane i-d (lanes below d keep their own value)
-template <typename T>
-__device__ __forceinline__ T shfl_up(T v, int d)
-{
-    return __shfl_up(v, d, kWave);
-}
-
-template <>
-__device__ __forceinline__ double2v shfl_up(double2v v, int d)
-{
-    return double2v{__shfl_up(v.x, d, kWave), __shfl_up(v.y, d, kWave)};
-}
-
-template <>
-__device__ __forceinline__ float2v shfl_up(float2v v, int d)
-{
-    return float2v{__shfl_up(v.x, d, kWave), __shfl_up(v.y, d, kWave)};
-}
-
 // Inclusive prefix sum of an int over the 64 lanes (DPP row shifts, then the
 // row broadcasts carry the running total across rows of 16).
 __device__ __forceinline__ int wave_incl_scan(int v, int /*lane*/)
@@ -201,11 +182,57 @@ __device__ __forceinline__ T wave_sum(T v)
     return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 
+// Place of 16-byte unit u in a tile's LDS product buffer of U units per lane:
+// u ^ swizzle_term<U>(u).  Products are written with consecutive lanes at
+// consecutive units (or pairs of units) and read with lane l at unit l*U + j;
+// XORing the low bits with higher ones spreads the reads over the banks: any 8
+// or 16 neighbouring lanes hit different 16-byte bank groups.
+template <int U>
+__device__ __forceinline__ int swizzle_term(int u)
+{
+    if constexpr (U == 2) return ((u >> 3) ^ (u >> 4)) & 1;
+    else if constexpr (U == 4) return ((u >> 3) ^ (u >> 5)) & 3;
+    else if constexpr (U == 8) return ((u >> 3) ^ (u >> 6)) & 7;
+    else return 0;
+}
+
+// v of lane (lane - d) mod 64.
+__device__ __forceinline__ int lane_back(int v, int lane, int d)
+{
+    return __builtin_amdgcn_ds_bpermute(lane * 4 + 256 - 4 * d, v);
+}
+
+__device__ __forceinline__ float lane_back(float v, int lane, int d)
+{
+    return __int_as_float(lane_back(__float_as_int(v), lane, d));
+}
+
+__device__ __forceinline__ double lane_back(double v, int lane, int d)
+{
+    union { double d; int i[2]; } u;
+    u.d = v;
+    u.i[0] = lane_back(u.i[0], lane, d);
+    u.i[1] = lane_back(u.i[1], lane, d);
+    return u.d;
+}
+
+__device__ __forceinline__ double2v lane_back(double2v v, int lane, int d)
+{
+    return double2v{lane_back(v.x, lane, d), lane_back(v.y, lane, d)};
+}
+
+__device__ __forceinline__ float2v lane_back(float2v v, int lane, int d)
+{
+    return float2v{lane_back(v.x, lane, d), lane_back(v.y, lane, d)};
+}
+
 // Segmented inclusive scan across lanes, left to right.  Lanes whose bit is
 // set in `head` start a new segment; lane 0 must be a head.  Returns, for lane
 // i, the sum of v over [s, i] where s is the last head at or before i.
 // Hillis-Steele doubling, stopping as soon as every lane's window reaches a
-// head (no step at all when every lane is a head).
+// head (no step at all when every lane is a head).  The windows' state is a
+// wave-uniform mask in scalar registers, each lane's bit of it the condition of
+// the select.
 template <typename T>
 __device__ __forceinline__ T wave_segscan(T v, uint64_t head, int lane)
 {
@@ -214,8 +241,9 @@ __device__ __forceinline__ T wave_segscan(T v, uint64_t head, int lane)
     for (int d = 1; d < kWave; d <<= 1) {
         if (cov == ~0ull) break;
         // lane i <- lane i-d (lane 0 is a head and never uses its value)
-        T up = d == 1 ? dpp<kDppWaveShr1>(v) : shfl_up(v, d);
-        if (!((cov >> lane) & 1ull)) v = up + v;
+        const T up = d == 1 ? dpp<kDppWaveShr1>(v) : lane_back(v, lane, d);
+        const T sum = up + v;
+        v = __builtin_amdgcn_inverse_ballot_w64(cov) ? v : sum;
         cov |= cov << d;
     }
     return v;
@@ -277,6 +305,32 @@ __device__ __forceinline__ double2v keep_or_zero(double2v v, bool keep)
 __device__ __forceinline__ float2v keep_or_zero(float2v v, bool keep)
 {
     return float2v{keep_or_zero(v.x, keep), keep_or_zero(v.y, keep)};
+}
+
+// +0 where the mask is all ones, v where it is 0 (bitwise, so that no branch or
+// compare stands between the sums of a lane).
+__device__ __forceinline__ double zero_where(double v, int mask)
+{
+    union { double d; int i[2]; } u;
+    u.d = v;
+    u.i[0] &= ~mask;
+    u.i[1] &= ~mask;
+    return u.d;
+}
+
+__device__ __forceinline__ float zero_where(float v, int mask)
+{
+    return __int_as_float(__float_as_int(v) & ~mask);
+}
+
+__device__ __forceinline__ double2v zero_where(double2v v, int mask)
+{
+    return double2v{zero_where(v.x, mask), zero_where(v.y, mask)};
+}
+
+__device__ __forceinline__ float2v zero_where(float2v v, int mask)
+{
+    return float2v{zero_where(v.x, mask), zero_where(v.y, mask)};
 }
 
 // Block index remap so that each XCD (blocks are dealt round-robin over the

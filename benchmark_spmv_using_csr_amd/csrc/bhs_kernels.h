@@ -400,6 +400,66 @@ struct XStage {
     }
 };
 
+// A tile's products (one value or a pair of right-hand sides each) through LDS:
+// written as loaded, G consecutive items per lane and load group, read back
+// lane-contiguous, item k of lane l being item l*S + k of the tile.
+template <typename T, int S, typename V>
+__device__ __forceinline__ void tile_transpose(V *sb, const V (&prod)[S], V (&pc)[S], int lane)
+{
+    constexpr int G = Tile<T, S>::G;
+    if constexpr (S == G) {                      // loaded lane-contiguous
+#pragma unroll
+        for (int k = 0; k < S; ++k) pc[k] = prod[k];
+        return;
+    }
+    constexpr int N = 16 / (int)sizeof(V);       // items per 16-byte unit
+    constexpr int U = S / N, H = G / N;          // units per lane, per lane and load group
+    typedef unsigned int bits_t __attribute__((ext_vector_type(4)));
+    bits_t *su = reinterpret_cast<bits_t *>(sb);
+#pragma unroll
+    for (int j = 0; j < S / G; ++j)
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            bits_t b;
+            __builtin_memcpy(&b, &prod[j * G + h * N], 16);
+            const int u = lane * H + h;
+            const int term = swizzle_term<U>(u) ^ swizzle_term<U>(j * kWave * H);
+            su[j * kWave * H + (u ^ term)] = b;
+        }
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const bits_t b = su[lane * U + (j ^ swizzle_term<U>(lane * U))];
+        __builtin_memcpy(&pc[j * N], &b, 16);
+    }
+    wave_sync();
+}
+
+// Lane-sequential segmented sums of a lane's items: at every head (bit k of hb:
+// item k starts a row) the sum before it is closed into sb, the lane's first one
+// at the place of the segment that the lanes before it leave open (lane 0, whose
+// item 0 always starts a segment, has none).  Returns the sum left open.
+template <typename V, int S>
+__device__ __forceinline__ V lane_segments(V *sb, const V (&pc)[S], unsigned hb, int seg_base,
+                                           int lane, V zero)
+{
+    V acc = zero;
+    int sidx = lane == 0 ? -1 : seg_base - 1;
+#pragma unroll
+    for (int kk = 0; kk < S; ++kk) {
+        const int h = __builtin_amdgcn_sbfe((int)hb, kk, 1);   // -1 at a head
+        if (kk == 0) {
+            if (h && lane > 0) sb[sidx] = zero;
+        } else if (h) {
+            sb[sidx] = acc;
+        }
+        sidx -= h;
+        acc = zero_where(acc, h);
+        acc += pc[kk];
+    }
+    return acc;
+}
+
 template <int R>
 struct RhsTag {
     static constexpr int value = R;
@@ -692,38 +752,18 @@ __device__ __forceinline__ void segsum_wave(const MatView<T> &mv, const int w, c
                     products(rt, xv, prod);
                     // products -> LDS in tile order, back lane-contiguous
                     wave_sync();
-    #pragma unroll
-                    for (int j = 0; j < S / G; ++j) {
-                        V *dst = sb + j * (kWave * G) + lane * G;
-    #pragma unroll
-                        for (int g = 0; g < G; ++g) dst[g] = prod[j * G + g];
-                    }
-                    wave_sync();
                     V pc[S];
-    #pragma unroll
-                    for (int kk = 0; kk < S; ++kk) pc[kk] = sb[lane * S + kk];
-                    wave_sync();
+                    tile_transpose<T, S>(sb, prod, pc, lane);
                     if (lane == 0 && cont) pc[0] = pc[0] + carry_getv(rt, rr);
 
                     // ---- lane-sequential segmented reduction -----------------
-                    V acc = zero, lead = zero;
-                    bool seen = false;
-                    int sidx = seg_base;
-    #pragma unroll
-                    for (int kk = 0; kk < S; ++kk) {
-                        if ((hb >> kk) & 1u) {
-                            if (seen) { sb[sidx] = acc; ++sidx; }
-                            else { lead = acc; seen = true; }
-                            acc = zero;
-                        }
-                        acc += pc[kk];
-                    }
+                    const V acc = lane_segments(sb, pc, hb, seg_base, lane, zero);
 
                     // ---- segments spanning lanes -----------------------------
-                    const uint64_t present = ballot(seen);  // bit 0 always set
+                    const uint64_t present = ballot(hb != 0u);   // bit 0 always set
                     const V I = wave_segscan(acc, present, lane);
                     const V Iprev = dpp<kDppWaveShr1>(I);     // lane i <- lane i-1 (lane 0: unused)
-                    if (seen && lane > 0) sb[seg_base - 1] = Iprev + lead;
+                    if (hb && lane > 0) sb[seg_base - 1] = Iprev + sb[seg_base - 1];
                     if (lane == kWave - 1) sb[K - 1] = I;
                     wave_sync();
 
@@ -909,61 +949,6 @@ struct TileShare {
     int kind[kMaxGroup];
 };
 
-// Place of 16-byte unit u in a tile's LDS product buffer (U units per lane).
-// A write has consecutive lanes at consecutive units, a read has lane l at unit
-// l*U + j; XORing the low bits with higher ones spreads both over the banks (any
-// 8 or 16 neighbouring lanes hit different 16-byte bank groups).
-template <int U>
-__device__ __forceinline__ int swizzle_term(int u)
-{
-    constexpr int b = U == 1 ? 0 : U == 2 ? 1 : U == 4 ? 2 : 3;
-    return ((u >> 3) ^ (u >> (3 + b))) & (U - 1);
-}
-
-// Segmented inclusive scan of wave_segscan (same sums) on scalar masks: whether
-// a lane adds at a step is its bit of a wave-uniform mask, used as the select's
-// condition directly.
-template <typename T>
-__device__ __forceinline__ T wave_segscan_masked(T v, uint64_t head, int lane)
-{
-    uint64_t cov = head;
-    const int la = lane * 4;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        if (cov == ~0ull) break;
-        T up;
-        if (d == 1) {
-            up = dpp<kDppWaveShr1>(v);
-        } else if constexpr (sizeof(T) == 8) {
-            union { T t; int i[2]; } a, b;
-            a.t = v;
-            b.i[0] = __builtin_amdgcn_ds_bpermute(la + 256 - 4 * d, a.i[0]);
-            b.i[1] = __builtin_amdgcn_ds_bpermute(la + 256 - 4 * d, a.i[1]);
-            up = b.t;
-        } else {
-            up = __int_as_float(__builtin_amdgcn_ds_bpermute(la + 256 - 4 * d, __float_as_int(v)));
-        }
-        const T sum = up + v;
-        v = __builtin_amdgcn_inverse_ballot_w64(cov) ? v : sum;
-        cov |= cov << d;
-    }
-    return v;
-}
-
-__device__ __forceinline__ double zero_where(double v, int mask)
-{
-    union { double d; int i[2]; } u;
-    u.d = v;
-    u.i[0] &= ~mask;
-    u.i[1] &= ~mask;
-    return u.d;
-}
-
-__device__ __forceinline__ float zero_where(float v, int mask)
-{
-    return __int_as_float(__float_as_int(v) & ~mask);
-}
-
 // Rows that cross logical waves, finished inside the launch.  The waves
 // first..last holding one row's nonzeros each send a partial; whoever comes
 // last adds them up, in the order of calibrate_window (wave order within
@@ -1064,9 +1049,16 @@ __device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first
     T tot = read_lane(wave_segscan(pv, 1ull << (e0 - base) | 1ull, lane), end);
     if (end == kWave - 1) {                 // up to a window's last entry: later windows follow
         T ext = T(0);
-        for (int nb = base + kWave; nb <= last; nb += kWave) {
-            const T pn = nb + lane <= last ? agent_load(part + nb + lane) : T(0);
-            ext = ext + wave_sum(pn);
+        for (int nb = base + kWave; nb <= last; nb += 4 * kWave) {   // four windows on their way at once
+            T pn[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int e = nb + i * kWave + lane;
+                pn[i] = e <= last ? agent_load(part + e) : T(0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (nb + i * kWave <= last) ext = ext + wave_sum(pn[i]);
         }
         tot = tot + ext;
     }
@@ -1139,9 +1131,7 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
     const SegsumParams<T> q)
 {
     constexpr int P = kWave * S;
-    constexpr int G = Tile<T, S>::G, U = S / G;
     constexpr int CR = CP * kWave;
-    typedef T unit_t __attribute__((ext_vector_type(G)));
     extern __shared__ double smem_raw[];
     const int lane = lane_id();
     int touch = 0;
@@ -1156,8 +1146,7 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
     const int g0 = wib & ~(TPW - 1);            // the logical wave's first tile in the block
     const int w = p >> __builtin_ctz(TPW);
     // product buffers first (16-byte aligned), then the head words, then the hand-over
-    unit_t *su = reinterpret_cast<unit_t *>(smem_raw) + wib * (kWave * U);
-    T *sb = reinterpret_cast<T *>(su);
+    T *sb = reinterpret_cast<T *>(smem_raw) + wib * P;
     unsigned *s_head = reinterpret_cast<unsigned *>(reinterpret_cast<T *>(smem_raw) + nwb * P) +
                        wib * kWave;
     TileShare<T> &sh = *reinterpret_cast<TileShare<T> *>(
@@ -1247,14 +1236,6 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
         // ---- bit flags
         bool lane_dirty = false;
         s_head[lane] = 0u;
-#pragma unroll
-        for (int j = 0; j < U; ++j) {                  // products in tile order
-            unit_t u;
-#pragma unroll
-            for (int g = 0; g < G; ++g) u[g] = prod[j * G + g];
-            const int term = swizzle_term<U>(lane) ^ swizzle_term<U>(j * kWave);
-            su[j * kWave + (lane ^ term)] = u;
-        }
         wave_sync();
         static_for<CP>([&](auto qc) {
             constexpr int qq = decltype(qc)::value;
@@ -1296,13 +1277,7 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
         wave_sync();
         hb = s_head[lane];
         if (lane == 0) hb |= 1u;
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-            const unit_t u = su[lane * U + (j ^ swizzle_term<U>(lane * U))];
-#pragma unroll
-            for (int g = 0; g < G; ++g) pc[j * G + g] = u[g];
-        }
-        wave_sync();
+        tile_transpose<T, S>(sb, prod, pc, lane);
         // ---- segment numbers
         const int nh = __popc(hb);
         const int incl = wave_incl_scan(nh, lane);
@@ -1311,23 +1286,9 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
         partial_tail = (r1 < q.m) && (rp_r1 < B + P);
         // the tile loop starts a logical wave with a carry of +0
         if (lane == 0 && cont && wib == g0) pc[0] = pc[0] + T(0);
-        // ---- lane-sequential segmented reduction: every head closes the sum
-        // before it, the lane's first one for the segment of the lanes before
-        int sidx = lane == 0 ? -1 : seg_base - 1;
-#pragma unroll
-        for (int kk = 0; kk < S; ++kk) {
-            const int h = __builtin_amdgcn_sbfe((int)hb, kk, 1);   // -1 at a head
-            if (kk == 0) {
-                if (h && lane > 0) sb[sidx] = T(0);
-            } else if (h) {
-                sb[sidx] = acc;
-            }
-            sidx -= h;
-            acc = zero_where(acc, h);
-            acc += pc[kk];
-        }
+        acc = lane_segments(sb, pc, hb, seg_base, lane, T(0));
         present = ballot(hb != 0u);
-        I = wave_segscan_masked(acc, present, lane);
+        I = wave_segscan(acc, present, lane);
         out_val = read_lane(I, kWave - 1);
     } else {
         T s = prod[0];
@@ -1381,7 +1342,7 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
                 if (hl) sb[0] = a0;
                 else acc = a0;
             }
-            I = wave_segscan_masked(acc, present, lane);
+            I = wave_segscan(acc, present, lane);
         }
         const T Iprev = dpp<kDppWaveShr1>(I);
         if (hb && lane > 0) sb[seg_base - 1] = Iprev + sb[seg_base - 1];
@@ -1614,6 +1575,287 @@ __global__ __launch_bounds__(512) void batched_kernel(
     }
 }
 
+// The same batch with one wave per tile (schedules of 1, 2, 4 or 8 tiles per
+// wave without x staging): a block is one (matrix, logical wave) item, its waves
+// the item's tiles, as in segsum_tiles_kernel.  The tile's stream, row boundaries
+// and flags are read and made once; then the right-hand sides pass in pairs (k
+// even, S * sizeof(T) <= 64 bytes; singly otherwise), the waves handing each
+// pair's open partials over through LDS behind one barrier a pair.
+//
+// batched_kernel holds the tile after this one and the pair after this one in
+// registers (176-256 VGPRs, 2 waves per SIMD, one right-hand side at a time
+// where pairs do not fit) and starts few waves for small matrices; here pairs
+// fit S = 8 in fp64 (156 VGPRs, 3 waves), and every tile has its wave at once.
+// The kernel waits for x lines (k = 16: a 128-byte line per nonzero and pair).
+// Replay of the graph, default schedule (S = 8, 4 tiles per wave), batched_kernel
+// -> this: 24 matrices of 1,000-87,000 rows (10M nonzeros, 145M products) fp64
+// 520 -> 249 us, fp32 341 -> 202; 24 of 1,000-4,000 rows 190 -> 47, 130 -> 42.
+template <typename V>
+struct BatchShare {
+    V val[2][kMaxGroup];       // by parity of the pass: a wave may be one pass ahead
+    int kind[kMaxGroup];       // bit 0: inside one row, bit 1: continues the row before it
+};
+
+template <typename T, int S, int KMAX>
+__global__ __launch_bounds__(512) void batched_tiles_kernel(
+    const int *__restrict__ row_ptr_all, const int *__restrict__ col_all,
+    const T *__restrict__ val_all, const T *__restrict__ x_all, T *__restrict__ y_all,
+    const int *__restrict__ tile_row_all, int *__restrict__ sync_row, T *__restrict__ sync_val,
+    int *__restrict__ sync_k, const BatchMeta *__restrict__ meta, const int2 *__restrict__ items,
+    int n_items, T alpha)
+{
+    constexpr int P = kWave * S, CP = 2, CR = CP * kWave;
+    constexpr bool kPairs = S * sizeof(T) <= 64;
+    using V2 = typename RhsVec<T, 2>::type;
+    extern __shared__ double smem_raw[];
+    const int lane = lane_id();
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int TPW = blockDim.x >> 6;
+    // 16 neighbouring items per XCD (blocks are dealt round-robin over the 8):
+    // they are mostly one matrix's neighbouring waves and share x lines in its L2
+    constexpr int kRun = 16;
+    int it = (int)blockIdx.x;
+    if ((it / (8 * kRun) + 1) * (8 * kRun) <= n_items)
+        it = it / (8 * kRun) * (8 * kRun) + (it % 8) * kRun + it / 8 % kRun;
+    const int2 iw = items[it];
+    const BatchMeta md = meta[iw.x];
+    const int w = iw.y, p = w * TPW + wib;
+    const int k = md.k;
+    const int *__restrict__ row_ptr = row_ptr_all + md.rp_off;
+    const int *__restrict__ tile_row = tile_row_all + md.tr_off;
+    const T *__restrict__ x = x_all + md.x_off;
+    T *__restrict__ y = y_all + md.y_off;
+    constexpr int kBuf = P * (kPairs ? 2 : 1);
+    T *s_buf = reinterpret_cast<T *>(smem_raw) + wib * kBuf;
+    unsigned *s_head =
+        reinterpret_cast<unsigned *>(reinterpret_cast<T *>(smem_raw) + TPW * kBuf) + wib * kWave;
+    unsigned char *s_share = reinterpret_cast<unsigned char *>(
+        reinterpret_cast<unsigned *>(reinterpret_cast<T *>(smem_raw) + TPW * kBuf) + TPW * kWave);
+    const bool active = p < md.NP;
+    const int pe = active ? p : 0;
+    const int B = pe * P;
+
+    Tile<T, S> t;
+    tile_load<T, S>(col_all + md.el_off, val_all + md.el_off, B, lane, t);
+    const int r0 = tile_row[pe], r1 = active ? tile_row[pe + 1] : r0;
+    const RowChunk<CP> cc = load_chunk<CP>(row_ptr, r0, lane, md.m);
+    const int rp_r1 = row_ptr[min(r1, md.m)];
+    if (md.lead_empty > 0 && active) {
+        const long long n = (long long)md.lead_empty * k;
+        const long long per = (n + md.NP - 1) / md.NP;
+        const long long hi = min((p + 1) * per, n);
+        for (long long r = p * per + lane; r < hi; r += kWave) y[r] = T(0);
+    }
+    const bool tail = B + P > md.nnz;
+    const bool general = r0 != r1;
+    const bool cont = read_lane(cc.a[0], 0) < B;
+    const int stop = (r1 == md.m) ? md.m - 1 : r1;
+    const bool big = r1 - r0 >= CR;
+    uint64_t mne[CP];
+    unsigned hb = 0;
+    bool dirty = false, partial_tail = false;
+    int seg_base = 0, K = 0;
+    uint64_t present = 1;
+    if (general) {
+        bool lane_dirty = false;
+        s_head[lane] = 0u;
+        wave_sync();
+        static_for<CP>([&](auto qc) {
+            constexpr int qq = decltype(qc)::value;
+            mne[qq] = 0ull;
+            if (qq > 0 && r0 + qq * kWave > stop) return;   // wave-uniform: no rows here
+            const bool have = r0 + qq * kWave + lane <= stop;
+            const bool ne = have && chunk_next<qq>(cc, lane) > cc.a[qq];
+            lane_dirty = lane_dirty || (have && !ne);
+            mne[qq] = ballot(ne);
+            const unsigned o = (unsigned)(cc.a[qq] - B);
+            if (ne && o < (unsigned)P) atomicOr(&s_head[o / S], 1u << (o % S));
+        });
+        if (big)
+            for (int rb = r0 + CR; rb <= stop;) {          // >= CR rows
+                const int rq = min(rb + lane, stop);
+                const int rp = row_ptr[rq], rpn = row_ptr[rq + 1];
+                const int vb = row_ptr[min(rb + kWave, stop + 1)];
+                if (rb + kWave <= stop && read_lane(rp, 0) == vb) {
+                    // 64 empty rows with more rows after them: skip the whole run
+                    const int re = empty_run_end(row_ptr, rb + kWave, vb, stop);
+                    lane_dirty = true;
+                    for (long long r = (long long)rb * k + lane; r < (long long)re * k; r += kWave)
+                        y[r] = T(0);
+                    rb = re;
+                    continue;
+                }
+                if (rb + lane <= stop) {
+                    const unsigned o = (unsigned)(rp - B);
+                    if (rpn > rp) {
+                        if (o < (unsigned)P) atomicOr(&s_head[o / S], 1u << (o % S));
+                    } else {
+                        lane_dirty = true;
+                        for (int rr = 0; rr < k; ++rr) y[(long long)(rb + lane) * k + rr] = T(0);
+                    }
+                }
+                rb += kWave;
+            }
+        dirty = ballot(lane_dirty) != 0ull;
+        wave_sync();
+        hb = s_head[lane];
+        if (lane == 0) hb |= 1u;
+        const int nh = __popc(hb);
+        const int incl = wave_incl_scan(nh, lane);
+        seg_base = incl - nh;
+        K = read_lane(incl, kWave - 1);
+        partial_tail = (r1 < md.m) && (rp_r1 < B + P);
+        present = ballot(hb != 0u);
+    }
+    const bool last = p == min((w + 1) * TPW, md.NP) - 1;
+    bool lead_open = cont;       // the row open at the item's start still is
+    int from = 0;                // the nearest earlier tile whose closing sum needs no carry
+
+    auto pass = [&](auto rt, int rr, int turn) __attribute__((always_inline)) {
+        constexpr int R = decltype(rt)::value;
+        using V = typename RhsVec<T, R>::type;
+        const V zero = static_cast<V>(T(0));
+        V *sb = reinterpret_cast<V *>(s_buf);
+        BatchShare<V> &sh = *reinterpret_cast<BatchShare<V> *>(s_share);
+        V acc = zero, I = zero, out_val, pc[S];
+        {
+            V prod[S];
+#pragma unroll
+            for (int kk = 0; kk < S; ++kk)
+                prod[kk] = *reinterpret_cast<const V *>(x + (long long)t.c[kk] * k + rr);
+#pragma unroll
+            for (int kk = 0; kk < S; ++kk) prod[kk] = t.v[kk] * prod[kk];
+            if (tail) {
+#pragma unroll
+                for (int kk = 0; kk < S; ++kk)
+                    prod[kk] = keep_or_zero(prod[kk], tile_item<T, S>(B, lane, kk) < md.nnz);
+            }
+            if (general) {
+                wave_sync();                 // the pass before has read its segments
+                tile_transpose<T, S>(sb, prod, pc, lane);
+                // the tile loop starts a logical wave with a carry of +0
+                if (lane == 0 && cont && wib == 0) pc[0] = pc[0] + zero;
+                acc = lane_segments(sb, pc, hb, seg_base, lane, zero);
+                I = wave_segscan(acc, present, lane);
+                out_val = read_lane(I, kWave - 1);
+            } else {
+                V s = prod[0];
+#pragma unroll
+                for (int kk = 1; kk < S; ++kk) s += prod[kk];
+                s = wave_sum(s);
+                out_val = (cont && wib == 0) ? zero + s : s;
+            }
+        }
+        V carry = zero;
+        const bool need = cont && wib > 0;
+        if (TPW > 1) {
+            if (lane == 0) {
+                sh.val[turn & 1][wib] = out_val;
+                if (turn == 0) sh.kind[wib] = (general ? 0 : 1) | (cont ? 2 : 0);
+            }
+            __syncthreads();
+            if (wib > 0) {
+                if (turn == 0) {
+                    const int kd = sh.kind[lane & (kMaxGroup - 1)];
+                    const unsigned fast = (unsigned)ballot(lane < kMaxGroup && (kd & 1));
+                    const unsigned conts = (unsigned)ballot(lane < kMaxGroup && (kd & 2));
+                    const unsigned below = (1u << wib) - 1;
+                    const unsigned stops = below & ~(fast & conts);
+                    from = stops ? 31 - __builtin_clz(stops) : 0;
+                    lead_open = (conts & 1u) && (below & ~fast) == 0;
+                }
+                carry = sh.val[turn & 1][from];
+                for (int j = from + 1; j < wib; ++j) carry = carry + sh.val[turn & 1][j];
+            }
+        }
+        if (!active) return;
+        auto store_y = [&](long long row, V v) {
+            *reinterpret_cast<V *>(y + row * k + rr) = v;
+        };
+        V *sv = reinterpret_cast<V *>(sync_val + (long long)(md.sync_off + w) * KMAX + rr);
+        if (general) {
+            if (need) {
+                // the carry starts lane 0's first sum: only the first segment changes
+                V a0 = pc[0] + carry;
+                const unsigned hl = hb & ~1u;
+#pragma unroll
+                for (int kk = 1; kk < S; ++kk) {
+                    const V n = a0 + pc[kk];
+                    if (!(hl & ((2u << kk) - 1))) a0 = n;
+                }
+                if (lane == 0) {
+                    if (hl) sb[0] = a0;
+                    else acc = a0;
+                }
+                I = wave_segscan(acc, present, lane);
+            }
+            const V Iprev = dpp<kDppWaveShr1>(I);
+            if (hb && lane > 0) sb[seg_base - 1] = Iprev + sb[seg_base - 1];
+            if (lane == kWave - 1) sb[K - 1] = I;
+            wave_sync();
+            const int kb = lead_open ? 1 : 0;
+            const int ke = partial_tail ? K - 1 : K;
+            if (!dirty) {
+                for (int kk = kb + lane; kk < ke; kk += kWave) store_y(r0 + kk, alpha * sb[kk]);
+            } else {
+                int running = 0;
+                static_for<CP>([&](auto qc) {
+                    constexpr int qq = decltype(qc)::value;
+                    if (qq > 0 && r0 + qq * kWave > stop) return;
+                    const int row = r0 + qq * kWave + lane;
+                    const bool ne = __builtin_amdgcn_inverse_ballot_w64(mne[qq]);
+                    const int rank = running + popc_below(mne[qq]);
+                    if (ne && rank >= kb && rank < ke) store_y(row, alpha * sb[rank]);
+                    else if (row <= stop && !ne) store_y(row, zero);
+                    running += __popcll(mne[qq]);
+                });
+                if (big)
+                    for (int rb = r0 + CR; rb <= stop;) {
+                        const int rq = min(rb + lane, stop);
+                        const int rp = row_ptr[rq], rpn = row_ptr[rq + 1];
+                        const int vb = row_ptr[min(rb + kWave, stop + 1)];
+                        if (rb + kWave <= stop && read_lane(rp, 0) == vb) {
+                            rb = empty_run_end(row_ptr, rb + kWave, vb, stop);   // no segments
+                            continue;
+                        }
+                        const int r = rb + lane;
+                        const bool ne = r <= stop && rpn > rp;
+                        const uint64_t msk = ballot(ne);
+                        const int rank = running + popc_below(msk);
+                        if (ne && rank >= kb && rank < ke) store_y(r, alpha * sb[rank]);
+                        running += __popcll(msk);
+                        rb += kWave;
+                    }
+            }
+            if (lane == 0) {
+                if (lead_open) *sv = alpha * sb[0];
+                if (last && partial_tail) store_y(r1, alpha * sb[K - 1]);
+            }
+        } else if (last && lane == 0) {
+            const V tot = alpha * (need ? carry + out_val : out_val);
+            if (lead_open) *sv = tot;
+            else store_y(r1, tot);
+        }
+    };
+    bool done = false;
+    if constexpr (kPairs) {
+        if ((k & 1) == 0) {
+            for (int rr = 0; rr < k; rr += 2) pass(RhsTag<2>{}, rr, rr >> 1);
+            done = true;
+        }
+    }
+    if (!done)
+        for (int rr = 0; rr < k; ++rr) pass(RhsTag<1>{}, rr, rr);
+    // the wave that closes (or passes on) a row from an earlier item says which
+    if (active && lane == 0) {
+        const bool sent = lead_open && (general || last);
+        if (sent || (wib == 0 && !cont)) {
+            sync_row[md.sync_off + w] = sent ? (int)md.y_off + (general ? r0 : r1) * k : -1;
+            sync_k[md.sync_off + w] = k;
+        }
+    }
+}
+
 // Calibration of a batch: sync entries of each matrix start on a multiple of
 // 64, so every window lies inside one matrix and matches the windows of that
 // matrix's own plain calibration; keys are y slots (unique across the batch).
@@ -1626,16 +1868,10 @@ __global__ __launch_bounds__(256) void calibrate_batched_kernel(const int *__res
     const int lane = lane_id();
     const int base = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kWave;
     if (base >= NW) return;
+    const int rr = (int)blockIdx.y;                // one right-hand side per grid row
     const int e = base + lane;
-    int kw = (e < NW && sync_row[e] >= 0) ? sync_k[e] : 0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const int o = __shfl_xor(kw, off, kWave);
-        kw = o > kw ? o : kw;
-    }
-    kw = __builtin_amdgcn_readfirstlane(kw);
-    for (int rr = 0; rr < kw; ++rr)
-        calibrate_window<T, KMAX>(sync_row, sync_val, sync_k, NW, base, rr, lane, y);
+    if (ballot(e < NW && sync_row[e] >= 0 && sync_k[e] > rr) == 0ull) return;
+    calibrate_window<T, KMAX>(sync_row, sync_val, sync_k, NW, base, rr, lane, y);
 }
 
 // y[i] = sum over panels p (in order) of row i's panel partial, +0 where row i

@@ -289,8 +289,10 @@ int bhs_d_batch_set_x(bhs_batch_t b, const double *const *X);
 int bhs_d_batch_set_schedule(bhs_batch_t b, const bhs_batch_schedule *s);
 int bhs_d_batch_get_schedule(bhs_batch_t b, bhs_batch_schedule *s);
 /* Y_i = alpha * A_i * X_i for every matrix: one hipGraph replay of
- * [queue reset] -> [persistent kernel over a global (matrix, tile range) queue]
- * -> [calibration].  Blocking. */
+ * [one block per (matrix, tile range)] -> [calibration] or, for schedules with
+ * x staging or other than 1, 2, 4 or 8 tiles per wave, of [queue reset] ->
+ * [persistent kernel over a global (matrix, tile range) queue] -> [calibration].
+ * waves_per_block and grid_blocks shape only the latter.  Blocking. */
 int bhs_d_batch_run(bhs_batch_t b, double alpha);
 /* The baseline: one plain SpMV (main kernel + calibration) per matrix per
  * right-hand side, back to back on one stream, on contiguous vectors. */

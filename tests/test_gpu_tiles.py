@@ -7,7 +7,7 @@ import pytest
 
 import cases
 import kernel_model as km
-from benchmark_spmv_using_csr_amd import _lib, matgen
+from benchmark_spmv_using_csr_amd import _lib, batched, matgen
 from benchmark_spmv_using_csr_amd.spmv import bhsparse_spmv
 from test_zz_no_alloc import DeviceArrays, call_noalloc
 
@@ -174,3 +174,31 @@ def test_more_logical_waves_than_the_fused_launch_takes(dtype):
     with DeviceArrays(A.row_ptr, A.col, v, x, np.full(A.m, np.nan, dtype)) as d:
         _lib.check(call_noalloc(dtype, A.m, A.n, A.nnz, d.ptrs, 1.5), "spmv_noalloc")
         assert np.array_equal(d.get(4, y), y)
+
+
+@pytest.mark.parametrize("S", [4, 8, 16])
+@pytest.mark.parametrize("T", [1, 2, 4, 8])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_batches_against_the_tile_loop(S, T, dtype):
+    """Even and odd numbers of right-hand sides over matrices whose rows meet tile
+    and wave ends every way, and the shapes with nothing to do, against one plain
+    SpMV (the tile loop) per matrix and right-hand side."""
+    cs = [cases.from_lengths(f"around {i}", lengths_around(64 * S, T, 6, 100 * S + 10 * T + i),
+                             n=4 * 64 * S * T + 100, seed=i) for i in range(4)]
+    cs += [cases.from_lengths("empty", [0] * 9, seed=1), cases.six_by_six(),
+           cases.from_lengths("lead", [0] * 3000 + [2] * 5, seed=2),
+           cases.from_lengths("one row", [5 * 64 * S * T + 3], seed=3)]
+    mats = [matgen.CSR(c.m, c.n, c.row_ptr, c.col, c.val.astype(dtype), c.name) for c in cs]
+    ks = [1, 2, 3, 16, 4, 5, 2, 16]
+    rng = np.random.default_rng(S * T)
+    Xs = [rng.uniform(-1, 1, (A.n, k)).astype(dtype) for A, k in zip(mats, ks)]
+    print(f"[gpu] batch S={S} T={T} {np.dtype(dtype).name}", flush=True)
+    b = batched.SpmvBatch(mats, ks, dtype)
+    b.set_schedule(S, T, 1, 0, 1, 0)
+    for turn in range(2):                       # the second run overwrites the first one's y
+        b.set_x([X * (turn + 1) for X in Xs])
+        b.run(0.75)
+        b.run_plain(0.75)
+        for i, (yb, yp) in enumerate(zip(b.y(), b.y(plain=True))):
+            assert np.array_equal(yb, yp), (i, mats[i].name, ks[i])
+    b.close()
