@@ -2081,6 +2081,29 @@ __global__ __launch_bounds__(256) void panel_scatter_kernel(
     }
 }
 
+// The right-hand sides of a batch one after another, for its per-vector
+// launches: xp[off + r * n + j] = x[off + j * k + r].  `per_mat` blocks a matrix;
+// a thread moves a column's k values, consecutive in x, and a wave's stores are
+// consecutive for each r.
+struct BatchX {
+    long long off;
+    int n, k;
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void rhs_major_kernel(const T *__restrict__ x, T *__restrict__ xp,
+                                                        const BatchX *__restrict__ bx, int n_mats,
+                                                        int per_mat)
+{
+    for (long long i = blockIdx.x / per_mat; i < n_mats; i += gridDim.x / per_mat) {
+        const BatchX b = bx[i];
+        for (long long j = (long long)(blockIdx.x % per_mat) * 256 + threadIdx.x; j < b.n;
+             j += (long long)per_mat * 256)
+            for (int r = 0; r < b.k; ++r)
+                xp[b.off + (long long)r * b.n + j] = x[b.off + j * b.k + r];
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void fill_kernel(T *__restrict__ p, long long n, T v)
 {
