@@ -651,6 +651,23 @@ int ensure_analysis(Impl<T> *im)
     return BHSPARSE_SUCCESS;
 }
 
+// Rows and nonzeros together from which a matrix is checked on the device, after
+// the upload: prepare_mem, host / device, 131k entries 181 / 202 us, 277k 265 /
+// 268, 1.1M 715 / 536, 11M 7.0 / 6.4 ms.
+constexpr long long kCheckOnDevice = 1 << 19;
+
+inline int not_monotone() { return set_error(BHSPARSE_INVALID_MATRIX, "row_ptr is not monotone"); }
+inline int bad_column() { return set_error(BHSPARSE_INVALID_MATRIX, "column index out of range"); }
+
+inline int check_csr(int m, int n, int nnz, const int *row_ptr, const int *col)
+{
+    for (int i = 0; i < m; i++)
+        if (row_ptr[i + 1] < row_ptr[i]) return not_monotone();
+    for (int j = 0; j < nnz; j++)
+        if (col[j] < 0 || col[j] >= n) return bad_column();
+    return BHSPARSE_SUCCESS;
+}
+
 template <typename T>
 int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const int *col,
               const T *val, const T *x, T *y)
@@ -665,12 +682,12 @@ int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const i
     if ((long long)nnz > kMaxNnz) return set_error(BHSPARSE_INVALID_MATRIX, "nnz too large");
     if (row_ptr[0] != 0 || row_ptr[m] != nnz)
         return set_error(BHSPARSE_INVALID_MATRIX, "row_ptr[0] must be 0 and row_ptr[m] == nnz");
-    for (int i = 0; i < m; i++)
-        if (row_ptr[i + 1] < row_ptr[i])
-            return set_error(BHSPARSE_INVALID_MATRIX, "row_ptr is not monotone");
-    for (int j = 0; j < nnz; j++)
-        if (col[j] < 0 || col[j] >= n)
-            return set_error(BHSPARSE_INVALID_MATRIX, "column index out of range");
+    // A handle with data keeps it when the new matrix is refused: there the host
+    // looks before anything is freed.
+    const bool on_device = !im->data && im->mem_mode == BHS_MEMORY_DEVICE &&
+                           (long long)m + nnz >= kCheckOnDevice;
+    if (!on_device)
+        if (int rc = check_csr(m, n, nnz, row_ptr, col)) return rc;
 
     release_data(im);
     BHS_HIP(hipSetDevice(im->device));
@@ -698,9 +715,12 @@ int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const i
     BHS_HIP(alloc_data(im, &im->d_y, sizeof(T) * (size_t)std::max(m, 1)));
     BHS_HIP(hipMemcpyAsync(im->d_row_ptr, row_ptr, sizeof(int) * ((size_t)m + 1),
                            hipMemcpyHostToDevice, im->stream));
-    BHS_HIP(hipMemsetAsync(im->d_col, 0, sizeof(int) * (size_t)im->nnz_pad, im->stream));
-    BHS_HIP(hipMemsetAsync(im->d_val, 0, sizeof(T) * (size_t)im->nnz_pad, im->stream));
-    BHS_HIP(hipMemsetAsync(im->d_x, 0, sizeof(T) * (size_t)std::max(n, 1), im->stream));
+    // past the last nonzero: column 0, value 0
+    BHS_HIP(hipMemsetAsync(im->d_col + nnz, 0, sizeof(int) * (size_t)(im->nnz_pad - nnz),
+                           im->stream));
+    BHS_HIP(hipMemsetAsync(im->d_val + nnz, 0, sizeof(T) * (size_t)(im->nnz_pad - nnz),
+                           im->stream));
+    if (n == 0) BHS_HIP(hipMemsetAsync(im->d_x, 0, sizeof(T), im->stream));
     if (nnz > 0) {
         BHS_HIP(hipMemcpyAsync(im->d_col, col, sizeof(int) * (size_t)nnz, hipMemcpyHostToDevice,
                                im->stream));
@@ -710,7 +730,20 @@ int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const i
     if (n > 0)
         BHS_HIP(hipMemcpyAsync(im->d_x, x, sizeof(T) * (size_t)n, hipMemcpyHostToDevice,
                                im->stream));
+    int bad = 0;
+    if (on_device) {
+        int *d_bad = reinterpret_cast<int *>(im->d_counters);
+        hipLaunchKernelGGL(bhs::fill_kernel<int>, dim3(1), dim3(64), 0, im->stream, d_bad, 1LL, 0);
+        hipLaunchKernelGGL(bhs::check_csr_kernel, dim3(1024), dim3(256), 0, im->stream,
+                           im->d_row_ptr, im->d_col, m, n, nnz, d_bad);
+        BHS_HIP(hipGetLastError());
+        BHS_HIP(hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, im->stream));
+    }
     BHS_HIP(hipStreamSynchronize(im->stream));
+    if (bad) {
+        release_data(im);
+        return bad & 1 ? not_monotone() : bad_column();
+    }
     im->h_y = y;
     im->data = true;
     return ensure_analysis(im);

@@ -2081,6 +2081,26 @@ __global__ __launch_bounds__(256) void panel_scatter_kernel(
     }
 }
 
+// Whether row_ptr is monotone (else *bad |= 1) and every column index lies in
+// [0, n) (else *bad |= 2): one read of row_ptr and col, col in 16-byte loads
+// (both from hipMalloc).
+__global__ __launch_bounds__(256) void check_csr_kernel(const int *__restrict__ row_ptr,
+                                                        const int *__restrict__ col, int m, int n,
+                                                        int nnz, int *__restrict__ bad)
+{
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x, step = (long long)gridDim.x * 256;
+    int b = 0;
+    for (long long i = t; i < m; i += step) b |= row_ptr[i + 1] < row_ptr[i];
+    const u32x4 *c4 = reinterpret_cast<const u32x4 *>(col);
+    const unsigned un = (unsigned)n;
+    for (long long i = t; i < nnz / 4; i += step) {
+        const u32x4 c = c4[i];
+        if (c.x >= un || c.y >= un || c.z >= un || c.w >= un) b |= 2;
+    }
+    if (t < nnz % 4 && (unsigned)col[nnz - 1 - t] >= un) b |= 2;
+    if (b) atomicOr(bad, b);
+}
+
 // The right-hand sides of a batch one after another, for its per-vector
 // launches: xp[off + r * n + j] = x[off + j * k + r].  `per_mat` blocks a matrix;
 // a thread moves a column's k values, consecutive in x, and a wave's stores are
