@@ -88,6 +88,8 @@ enum ValueKind { kFloat = 1, kDouble = 2 };
 // that also finishes the rows crossing logical waves (one kernel in all).
 enum SegsumKernel { kWaveLoop, kTilePerWave, kTilePerWaveFused };
 
+#include "bhs_stage.inc"
+
 template <typename T>
 struct Impl {
     int device = -1;
@@ -226,6 +228,7 @@ int init_platform(bhs_handle_t h, int device)
         BHS_HIP(hipEventCreateWithFlags(&im->done, hipEventDisableTiming));
         BHS_HIP(hipMalloc(&im->d_counters, 8 * sizeof(unsigned long long)));
     }
+    if (!im->platform) stage_pool().attach();
     im->device = device;
     im->platform = true;
     void *sp[2];                     // the device's scratch addresses, looked up once
@@ -715,8 +718,9 @@ int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const i
     BHS_HIP(alloc_data(im, &im->d_val, sizeof(T) * (size_t)im->nnz_pad));
     BHS_HIP(alloc_data(im, &im->d_x, sizeof(T) * (size_t)std::max(n, 1)));
     BHS_HIP(alloc_data(im, &im->d_y, sizeof(T) * (size_t)std::max(m, 1)));
-    BHS_HIP(hipMemcpyAsync(im->d_row_ptr, row_ptr, sizeof(int) * ((size_t)m + 1),
-                           hipMemcpyHostToDevice, im->stream));
+    StageLease lease(im->stream, im->data_mode == BHS_MEMORY_DEVICE);
+    if (int rc = upload(lease, im->stream, im->d_row_ptr, row_ptr, sizeof(int) * ((size_t)m + 1)))
+        return rc;
     // past the last nonzero: column 0, value 0
     BHS_HIP(hipMemsetAsync(im->d_col + nnz, 0, sizeof(int) * (size_t)(im->nnz_pad - nnz),
                            im->stream));
@@ -724,14 +728,11 @@ int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const i
                            im->stream));
     if (n == 0) BHS_HIP(hipMemsetAsync(im->d_x, 0, sizeof(T), im->stream));
     if (nnz > 0) {
-        BHS_HIP(hipMemcpyAsync(im->d_col, col, sizeof(int) * (size_t)nnz, hipMemcpyHostToDevice,
-                               im->stream));
-        BHS_HIP(hipMemcpyAsync(im->d_val, val, sizeof(T) * (size_t)nnz, hipMemcpyHostToDevice,
-                               im->stream));
+        if (int rc = upload(lease, im->stream, im->d_col, col, sizeof(int) * (size_t)nnz)) return rc;
+        if (int rc = upload(lease, im->stream, im->d_val, val, sizeof(T) * (size_t)nnz)) return rc;
     }
     if (n > 0)
-        BHS_HIP(hipMemcpyAsync(im->d_x, x, sizeof(T) * (size_t)n, hipMemcpyHostToDevice,
-                               im->stream));
+        if (int rc = upload(lease, im->stream, im->d_x, x, sizeof(T) * (size_t)n)) return rc;
     int bad = 0;
     if (on_device) {
         int *d_bad = reinterpret_cast<int *>(im->d_counters);
@@ -742,6 +743,8 @@ int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const i
         BHS_HIP(hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, im->stream));
     }
     BHS_HIP(hipStreamSynchronize(im->stream));
+    if (lease)
+        if (int rc = lease.finish()) return rc;
     if (bad) {
         release_data(im);
         return bad & 1 ? not_monotone() : bad_column();
@@ -759,9 +762,14 @@ int set_x(bhs_handle_t h, const T *x)
     if (!im->data) return set_error(BHSPARSE_NOT_INITIALIZED, "init_data first");
     if (im->n > 0 && !x) return set_error(BHSPARSE_INVALID_ARGUMENT, "null x");
     BHS_HIP(hipSetDevice(im->device));
+    const size_t bytes = sizeof(T) * (size_t)im->n;
+    StageLease lease(im->stream, im->n > 0 && im->data_mode == BHS_MEMORY_DEVICE && pageable(x));
+    if (lease) {
+        if (int rc = lease.write(im->d_x, x, bytes)) return rc;
+        return lease.finish();
+    }
     if (im->n > 0)
-        BHS_HIP(hipMemcpyAsync(im->d_x, x, sizeof(T) * (size_t)im->n, hipMemcpyHostToDevice,
-                               im->stream));
+        BHS_HIP(hipMemcpyAsync(im->d_x, x, bytes, hipMemcpyHostToDevice, im->stream));
     BHS_HIP(hipStreamSynchronize(im->stream));
     return BHSPARSE_SUCCESS;
 }
@@ -1106,9 +1114,14 @@ int get_y_to(bhs_handle_t h, T *out)
     if (!im->data) return set_error(BHSPARSE_NOT_INITIALIZED, "init_data first");
     if (im->m > 0 && !out) return set_error(BHSPARSE_INVALID_ARGUMENT, "null y");
     BHS_HIP(hipSetDevice(im->device));
+    const size_t bytes = sizeof(T) * (size_t)im->m;
+    StageLease lease(im->stream, im->m > 0 && im->data_mode == BHS_MEMORY_DEVICE && pageable(out));
+    if (lease)
+        return lease.read(im->d_y, bytes, [&](size_t o, const char *p, size_t len) {
+            copy_part(reinterpret_cast<char *>(out) + o, p, len, bytes >= kPastCaches);
+        });
     if (im->m > 0)
-        BHS_HIP(hipMemcpyAsync(out, im->d_y, sizeof(T) * (size_t)im->m, hipMemcpyDeviceToHost,
-                               im->stream));
+        BHS_HIP(hipMemcpyAsync(out, im->d_y, bytes, hipMemcpyDeviceToHost, im->stream));
     BHS_HIP(hipStreamSynchronize(im->stream));
     return BHSPARSE_SUCCESS;
 }
@@ -1153,6 +1166,7 @@ int free_platform(bhs_handle_t h)
         if (e) { (void)hipEventDestroy(e); e = nullptr; }
     if (im->done) (void)hipEventDestroy(im->done);
     im->done = nullptr;
+    stage_pool().detach();
     if (im->stream) (void)hipStreamDestroy(im->stream);
     im->stream = nullptr;
     im->platform = false;

@@ -2081,6 +2081,46 @@ __global__ __launch_bounds__(256) void panel_scatter_kernel(
     }
 }
 
+// Copies `words` 32-bit words in pieces of kPieceBytes, one end of the copy pinned
+// host memory, and sets flags[p * flag_step] = tag behind piece p: to the host, when
+// its data are there; from the host, when they have been read (what follows on the
+// stream finds them; a release to the system here would write the L2 back, 15 us).
+// Blocks take the pieces in turn, so they are done in about their order.  src
+// and dst on 16 bytes.  (32-bit sizes on purpose: with min() of two signed 64-bit
+// uniform values the compiler's code took a stale condition and copied whole pieces.)
+constexpr int kPieceBytes = 16384;
+
+template <bool TO_HOST>
+__global__ __launch_bounds__(256) void copy_pieces_kernel(const unsigned *__restrict__ src,
+                                                          unsigned *__restrict__ dst, int words,
+                                                          unsigned *flags, int flag_step,
+                                                          unsigned tag)
+{
+    constexpr int W = kPieceBytes / 4;
+    for (int p = blockIdx.x; p * W < words; p += gridDim.x) {
+        const unsigned *s = src + p * W;
+        unsigned *d = dst + p * W;
+        const int n = min(words - p * W, W);
+        u32x4 v[W / 1024];                // all of a thread's loads on their way at once
+#pragma unroll
+        for (int i = 0; i < W / 1024; ++i) {
+            const int at = i * 256 + (int)threadIdx.x;
+            if (at < n / 4) v[i] = reinterpret_cast<const u32x4 *>(s)[at];
+        }
+#pragma unroll
+        for (int i = 0; i < W / 1024; ++i) {
+            const int at = i * 256 + (int)threadIdx.x;
+            if (at < n / 4) reinterpret_cast<u32x4 *>(d)[at] = v[i];
+        }
+        if ((int)threadIdx.x < n % 4) d[n / 4 * 4 + threadIdx.x] = s[n / 4 * 4 + threadIdx.x];
+        if constexpr (TO_HOST) __threadfence_system();
+        __syncthreads();                  // every wave's data are there, or read
+        if (threadIdx.x == 0)
+            __hip_atomic_store(flags + p * flag_step, tag, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // Whether row_ptr is monotone (else *bad |= 1) and every column index lies in
 // [0, n) (else *bad |= 2): one read of row_ptr and col, col in 16-byte loads
 // (both from hipMalloc).

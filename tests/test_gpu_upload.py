@@ -1,9 +1,12 @@
-"""Upload of A: a matrix large enough to be checked on the device is refused for
-the same faults, with the same codes, as one checked on the host."""
+"""Copies between host and device: a matrix large enough to be checked on the
+device is refused for the same faults, with the same codes, as one checked on the
+host; x and y arrive whole by every route (staged or not, several threads)."""
+import threading
+
 import numpy as np
 import pytest
 
-from benchmark_spmv_using_csr_amd import matgen
+from benchmark_spmv_using_csr_amd import batched, matgen
 from benchmark_spmv_using_csr_amd._lib import (BHSPARSE_INVALID_MATRIX, BHSPARSE_NOT_INITIALIZED,
                                                spmv_lib)
 from benchmark_spmv_using_csr_amd.spmv import bhsparse_spmv
@@ -53,3 +56,73 @@ def test_a_bad_matrix_is_refused(rows, what, loaded):
         assert np.all(np.abs(y - want) <= 32 * np.finfo(np.float64).eps * scale)
     finally:
         op.close()
+
+
+def _identity(n):
+    return matgen.CSR(n, n, np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32),
+                      np.ones(n))
+
+
+def _round_trips(n, dtype, seed, times):
+    """x through set_x, a diagonal matrix and get_y: exact, by value."""
+    A, rng = _identity(n), np.random.default_rng(seed)
+    op = bhsparse_spmv(dtype)
+    try:
+        assert op.init_platform(0) == 0
+        y = np.zeros(n + 3, dtype)                   # three guards behind y
+        y[n:] = 7
+        x = rng.random(n).astype(dtype)
+        assert op.prepare_mem(n, n, n, A.row_ptr, A.col, A.val.astype(dtype), x, y) == 0
+        assert op.spmv(1.0) == 0 and op.get_y() == 0
+        ok = np.array_equal(y[:n], x)
+        for _ in range(times):
+            x = rng.random(n).astype(dtype)
+            assert op.set_x(x) == 0
+            x2 = x.copy()
+            x[:] = 0                                 # the call has read x when it returns
+            assert op.spmv(1.0) == 0 and op.get_y() == 0
+            ok = ok and np.array_equal(y[:n], x2)
+        return ok and bool(np.all(y[n:] == 7))
+    finally:
+        op.close()
+
+
+# 16 KB pieces, chunks of 256 KB and 1 MB, the two halves of 2 MB, the reuse of the ring
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("words", [2, 6, 1022, 4094, 4096, 4098, 8200, 32766, 65534, 65536,
+                                   65538, 262146, 524286, 524290, 1048578, 2097152, 2097154, 5000002])
+def test_x_and_y_arrive(words, dtype):
+    assert _round_trips(words // (np.dtype(dtype).itemsize // 4), dtype, words, 3)
+
+
+def test_x_and_y_arrive_in_threads():
+    """More threads than pinned buffers, both directions."""
+    sizes = [33, 4000, 16_000, 300_000, 700_001, 5]
+    out = [None] * len(sizes)
+
+    def work(i):
+        out[i] = _round_trips(sizes[i], np.float64, i, 20)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert out == [True] * len(sizes)
+
+
+@pytest.mark.parametrize("sizes", [[1, 40, 0, 7], [3000, 17_000, 64], [9000] * 40, [300_000, 5, 90_001]])
+def test_batch_x_and_y_arrive(sizes):
+    rng = np.random.default_rng(len(sizes))
+    ks = [(1, 4, 16, 3)[i % 4] for i in range(len(sizes))]
+    b = batched.SpmvBatch([_identity(n) for n in sizes], ks, np.float64)
+    try:
+        for _ in range(3):
+            X = [rng.random((n, k)) for n, k in zip(sizes, ks)]
+            b.set_x(X)
+            b.run(1.0)
+            assert all(np.array_equal(g, x) for g, x in zip(b.y(), X))
+            b.run_plain(1.0)
+            assert all(np.array_equal(g, x) for g, x in zip(b.y(plain=True), X))
+    finally:
+        b.close()
