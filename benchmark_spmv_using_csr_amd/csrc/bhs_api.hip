@@ -151,7 +151,7 @@ struct Impl {
     // ev[0]/ev[2]: recorded around a whole call; ev[1]/ev[3]: attached to the
     // main kernel's dispatch (hipExtLaunchKernelGGL), its exact duration
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    hipEvent_t done = nullptr;                  // completion of a blocking call
+    Signal signal;                              // of the end of a blocking call
     size_t max_lds = 65536;   // per-block LDS limit of a configuration
     size_t dev_lds = 65536;   // per-block LDS limit of the device
 };
@@ -225,10 +225,9 @@ int init_platform(bhs_handle_t h, int device)
     if (!im->platform) {
         BHS_HIP(hipStreamCreateWithFlags(&im->stream, hipStreamNonBlocking));
         for (auto &e : im->ev) BHS_HIP(create_timing_event(&e));
-        BHS_HIP(hipEventCreateWithFlags(&im->done, hipEventDisableTiming));
         BHS_HIP(hipMalloc(&im->d_counters, 8 * sizeof(unsigned long long)));
     }
-    if (!im->platform) stage_pool().attach();
+    if (!im->platform) stage_pool().attach(im->signal);
     im->device = device;
     im->platform = true;
     void *sp[2];                     // the device's scratch addresses, looked up once
@@ -909,38 +908,26 @@ void launch_segsum(Impl<T> *im, T alpha, unsigned long long *stats, hipEvent_t e
 }
 
 template <typename T>
-void launch_calibrate(Impl<T> *im, hipEvent_t done = nullptr)
+void launch_calibrate(Impl<T> *im)
 {
     const int threads = 256;
-    const dim3 grid((im->NW + threads - 1) / threads);
-    if (done)
-        hipExtLaunchKernelGGL(bhs::calibrate_kernel<T>, grid, dim3(threads), 0u, im->stream,
-                              nullptr, done, 0u, (const int *)im->d_sync_row,
-                              (const T *)im->d_sync_val, im->NW, active_layout(im).y);
-    else
-        hipLaunchKernelGGL(bhs::calibrate_kernel<T>, grid, dim3(threads), 0, im->stream,
-                           im->d_sync_row, im->d_sync_val, im->NW, active_layout(im).y);
+    hipLaunchKernelGGL(bhs::calibrate_kernel<T>, dim3((im->NW + threads - 1) / threads),
+                       dim3(threads), 0, im->stream, im->d_sync_row, im->d_sync_val, im->NW,
+                       active_layout(im).y);
 }
 
 template <typename T>
-void launch_combine(Impl<T> *im, hipEvent_t done = nullptr)
+void launch_combine(Impl<T> *im)
 {
     constexpr int kGroups = bhs::kCombineGroups;   // 64-row groups per wave
     const int threads = 256;
     const long long rows_per_block = 64LL * kGroups * (threads / 64);
     const long long blocks = ((long long)im->m + rows_per_block - 1) / rows_per_block;
     auto go = [&](auto kern) {
-        if (done)
-            hipExtLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(threads), 0u, im->stream,
-                                  nullptr, done, 0u, (const T *)im->d_ystack,
-                                  (const unsigned char *)im->d_pmask, (const int *)im->d_pbase,
-                                  im->m, im->d_y, (const bhs::ChainRec *)im->d_chains,
-                                  (const T *)im->d_sync_val);
-        else
-            hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(threads), 0, im->stream,
-                               (const T *)im->d_ystack, (const unsigned char *)im->d_pmask,
-                               (const int *)im->d_pbase, im->m, im->d_y,
-                               (const bhs::ChainRec *)im->d_chains, (const T *)im->d_sync_val);
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(threads), 0, im->stream,
+                           (const T *)im->d_ystack, (const unsigned char *)im->d_pmask,
+                           (const int *)im->d_pbase, im->m, im->d_y,
+                           (const bhs::ChainRec *)im->d_chains, (const T *)im->d_sync_val);
     };
     switch (im->pan_n) {
     case 2: go(bhs::combine_panels_kernel<T, 2, kGroups>); break;
@@ -1015,12 +1002,10 @@ size_t segsum_lds_bytes(const bhs_config &c)
 
 // Enqueues one y = alpha*A*x.  If main_start and main_done are given they are
 // attached to the main kernel's dispatch and time exactly that kernel (they
-// are recorded around the fill when there is no kernel to time).  `done` is
-// complete when the whole call is: attached to its last kernel's dispatch, or
-// recorded behind it.
+// are recorded around the fill when there is no kernel to time).
 template <typename T>
 int enqueue_spmv(Impl<T> *im, T alpha, hipEvent_t main_start = nullptr,
-                 hipEvent_t main_done = nullptr, hipEvent_t done = nullptr)
+                 hipEvent_t main_done = nullptr)
 {
     if (!im->data) return set_error(BHSPARSE_NOT_INITIALIZED, "init_data first");
     if (int rc = ensure_analysis(im)) return rc;
@@ -1030,11 +1015,10 @@ int enqueue_spmv(Impl<T> *im, T alpha, hipEvent_t main_start = nullptr,
             BHS_HIP(hipEventRecord(main_start, im->stream));
             BHS_HIP(hipEventRecord(main_done, im->stream));
         }
-        if (done) BHS_HIP(hipEventRecord(done, im->stream));
         return BHSPARSE_SUCCESS;
     }
     if (im->cfg.variant == BHS_VARIANT_CSRVEC) {
-        launch_csrvec(im, alpha, main_start, done ? done : main_done);
+        launch_csrvec(im, alpha, main_start, main_done);
         BHS_HIP(hipGetLastError());
         return BHSPARSE_SUCCESS;
     }
@@ -1043,7 +1027,6 @@ int enqueue_spmv(Impl<T> *im, T alpha, hipEvent_t main_start = nullptr,
         launch_fill(im, im->d_y, im->m);
         BHS_HIP(hipGetLastError());
         if (timed) BHS_HIP(hipEventRecord(main_done, im->stream));
-        if (done) BHS_HIP(hipEventRecord(done, im->stream));
         return BHSPARSE_SUCCESS;
     }
     if (segsum_lds_bytes<T>(im->cfg) > im->max_lds)
@@ -1053,12 +1036,11 @@ int enqueue_spmv(Impl<T> *im, T alpha, hipEvent_t main_start = nullptr,
     // a boundary partial
     const bool combine = im->cfg.variant == BHS_VARIANT_SEGSUM_PANELS;
     const bool calibrate = !combine && im->kernel != kTilePerWaveFused && im->NW > 1;
-    const hipEvent_t last = done && !combine && !calibrate ? done : main_done;
-    if (im->kernel == kWaveLoop) launch_segsum<T, false>(im, alpha, nullptr, main_start, last);
-    else launch_tiles(im, alpha, main_start, last);
+    if (im->kernel == kWaveLoop) launch_segsum<T, false>(im, alpha, nullptr, main_start, main_done);
+    else launch_tiles(im, alpha, main_start, main_done);
     BHS_HIP(hipGetLastError());
-    if (calibrate) launch_calibrate(im, done);
-    if (combine) launch_combine(im, done);
+    if (calibrate) launch_calibrate(im);
+    if (combine) launch_combine(im);
     BHS_HIP(hipGetLastError());
     return BHSPARSE_SUCCESS;
 }
@@ -1091,19 +1073,8 @@ int spmv(bhs_handle_t h, T alpha)
     if (int rc = get_impl(h, &im)) return rc;
     if (!im->platform) return set_error(BHSPARSE_NOT_INITIALIZED, "init_platform first");
     BHS_HIP(hipSetDevice(im->device));
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    BHS_HIP(hipStreamIsCapturing(im->stream, &cap));
-    if (im->data_mode != BHS_MEMORY_DEVICE || cap != hipStreamCaptureStatusNone) {
-        if (int rc = enqueue_spmv(im, alpha)) return rc;
-        BHS_HIP(hipStreamSynchronize(im->stream));
-        return BHSPARSE_SUCCESS;
-    }
-    // waiting for the last kernel's own completion signal spares the marker that
-    // hipStreamSynchronize puts behind it: 18.6 -> 16.1 us for a kernel of 8.4
-    if (int rc = enqueue_spmv(im, alpha, (hipEvent_t) nullptr, (hipEvent_t) nullptr, im->done))
-        return rc;
-    BHS_HIP(hipEventSynchronize(im->done));
-    return BHSPARSE_SUCCESS;
+    if (int rc = enqueue_spmv(im, alpha)) return rc;
+    return reach(im->stream, im->data_mode == BHS_MEMORY_DEVICE ? &im->signal : nullptr);
 }
 
 template <typename T>
@@ -1164,9 +1135,7 @@ int free_platform(bhs_handle_t h)
     free_ptr(im->d_tuner_scores);
     for (auto &e : im->ev)
         if (e) { (void)hipEventDestroy(e); e = nullptr; }
-    if (im->done) (void)hipEventDestroy(im->done);
-    im->done = nullptr;
-    stage_pool().detach();
+    stage_pool().detach(im->signal);
     if (im->stream) (void)hipStreamDestroy(im->stream);
     im->stream = nullptr;
     im->platform = false;

@@ -2121,6 +2121,12 @@ __global__ __launch_bounds__(256) void copy_pieces_kernel(const unsigned *__rest
     }
 }
 
+// Tells the host that the stream has come here.
+__global__ void signal_kernel(unsigned *flag, unsigned tag)
+{
+    __hip_atomic_store(flag, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Whether row_ptr is monotone (else *bad |= 1) and every column index lies in
 // [0, n) (else *bad |= 2): one read of row_ptr and col, col in 16-byte loads
 // (both from hipMalloc).

@@ -126,3 +126,24 @@ def test_batch_x_and_y_arrive(sizes):
             assert all(np.array_equal(g, x) for g, x in zip(b.y(plain=True), X))
     finally:
         b.close()
+
+
+def test_more_handles_than_signal_words():
+    """258 open handles: the last ones wait by synchronising their stream."""
+    A = _identity(10)
+    ops, ys = [], []
+    try:
+        for i in range(258):
+            op = bhsparse_spmv(np.float64)
+            ops.append(op)
+            ys.append(np.zeros(10))
+            assert op.init_platform(0) == 0
+            x = np.arange(10) + i + 1.0
+            assert op.prepare_mem(10, 10, 10, A.row_ptr, A.col, A.val, x, ys[-1]) == 0
+        for _ in range(2):
+            for i, op in enumerate(ops):
+                assert op.spmv(2.0) == 0 and op.get_y() == 0
+                assert np.array_equal(ys[i], 2 * (np.arange(10) + i + 1.0))
+    finally:
+        for op in ops:
+            op.close()
