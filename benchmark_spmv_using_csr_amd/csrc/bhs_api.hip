@@ -563,10 +563,11 @@ size_t tile_lds_bytes(int S, int waves)
 //    uniform rows 10.7 / 9.1, band of 41 8.4 / 6.1, power law with one row
 //    over 390 waves 12.3 / 13.3; 2M (7.8k), power law 22.2 / 22.7.
 //  * fp32, S = 4 (2 KB of A a wave), T = 4, Laplacian 160^3: 63.9 / 70.8 warm.
-//  * T > 1 with up to 32 logical waves (65,000 nonzeros at the default tile)
-//    stays on the loop, 14 us against 6: the fixed default tile is the yardstick
-//    of the tuner's speedup (at least 1.2 over its test set), and what such a
-//    matrix should run is the tuner's csr-vector (4.4 us) or one tile per wave.
+//  * T > 1 with up to 24 logical waves (49,000 nonzeros at the default tile)
+//    stays on the loop, 13 us against 5.6: the fixed default tile is the yardstick
+//    of the tuner's speedup (at least 1.2 over its test set: 1.10 without this
+//    line, 1.18 with 16, 1.23 with 24), and what such a matrix should run is the
+//    tuner's csr-vector (4.4 us) or one tile per wave.
 // Shapes the one-wave-per-tile kernel is not built for (T not a power of two
 // up to 8, S = 32) and blocks beyond the device's LDS take the loop.
 template <typename T>
@@ -577,7 +578,7 @@ SegsumKernel pick_kernel(const Impl<T> *im, long long NW)
     if (c.variant != BHS_VARIANT_SEGSUM || S > 16 || TPW > bhs::kMaxGroup || (TPW & (TPW - 1)))
         return kWaveLoop;
     if (tile_lds_bytes<T>(S, tile_block_waves(c)) > im->dev_lds) return kWaveLoop;
-    if (TPW > 1 && NW <= 32) return kWaveLoop;
+    if (TPW > 1 && NW <= 24) return kWaveLoop;
     if (NW <= (TPW == 1 || S == 4 ? 4096 : 16384)) return kTilePerWaveFused;
     return TPW == 1 || S * sizeof(T) < 32 ? kWaveLoop : kTilePerWave;
 }
