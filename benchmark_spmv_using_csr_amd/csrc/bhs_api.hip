@@ -600,7 +600,10 @@ int ensure_analysis(Impl<T> *im)
     const int P = 64 * im->cfg.items_per_lane;
     const int TPW = im->cfg.tiles_per_wave;
     const int layout = im->cfg.variant == BHS_VARIANT_SEGSUM_PANELS ? im->cfg.tpv : 0;
-    if (im->an_P == P && im->an_TPW == TPW && im->an_layout == layout) return BHSPARSE_SUCCESS;
+    if (im->an_P == P && im->an_TPW == TPW && im->an_layout == layout) {
+        im->kernel = pick_kernel(im, im->NW);   // csr-vector and plain classes share a partition
+        return BHSPARSE_SUCCESS;
+    }
     if (layout > 0 && im->m > 0)
         if (int rc = build_panels(im, layout)) return rc;
     const Layout<T> L = active_layout(im);
