@@ -1214,10 +1214,9 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
     else if (lead_empty < 0)
         lead_empty = tile_row[0];
     if (lead_empty > 0 && active) {
-        const unsigned per = ((unsigned)lead_empty + (unsigned)q.NP - 1) / (unsigned)q.NP;
-        const long long lo = (long long)p * per;
-        const long long hi = min(lo + per, (long long)lead_empty);
-        for (long long r = lo + lane; r < hi; r += kWave) y[r] = T(0);
+        const unsigned n = (unsigned)lead_empty, per = (n + (unsigned)q.NP - 1) / (unsigned)q.NP;
+        const unsigned lo = (unsigned)p * per;               // at most n + NP
+        for (unsigned r = lo + lane; r < lo + per && r < n; r += kWave) y[r] = T(0);
     }
 
     const bool general = r0 != r1;
@@ -1641,10 +1640,9 @@ __global__ __launch_bounds__(512) void batched_tiles_kernel(
     const RowChunk<CP> cc = load_chunk<CP>(row_ptr, r0, lane, md.m);
     const int rp_r1 = row_ptr[min(r1, md.m)];
     if (md.lead_empty > 0 && active) {
-        const long long n = (long long)md.lead_empty * k;
-        const long long per = (n + md.NP - 1) / md.NP;
-        const long long hi = min((p + 1) * per, n);
-        for (long long r = p * per + lane; r < hi; r += kWave) y[r] = T(0);
+        const unsigned n = (unsigned)md.lead_empty * k;      // a batch's y is below 2^31
+        const unsigned per = (n + (unsigned)md.NP - 1) / (unsigned)md.NP, lo = (unsigned)p * per;
+        for (unsigned r = lo + lane; r < lo + per && r < n; r += kWave) y[r] = T(0);
     }
     const bool tail = B + P > md.nnz;
     const bool general = r0 != r1;
@@ -2086,8 +2084,7 @@ __global__ __launch_bounds__(256) void panel_scatter_kernel(
 // its data are there; from the host, when they have been read (what follows on the
 // stream finds them; a release to the system here would write the L2 back, 15 us).
 // Blocks take the pieces in turn, so they are done in about their order.  src
-// and dst on 16 bytes.  (32-bit sizes on purpose: with min() of two signed 64-bit
-// uniform values the compiler's code took a stale condition and copied whole pieces.)
+// and dst on 16 bytes; a launch moves 2 MB at most, so 32-bit sizes do.
 constexpr int kPieceBytes = 16384;
 
 template <bool TO_HOST>

@@ -202,3 +202,54 @@ def test_batches_against_the_tile_loop(S, T, dtype):
         for i, (yb, yp) in enumerate(zip(b.y(), b.y(plain=True))):
             assert np.array_equal(yb, yp), (i, mats[i].name, ks[i])
     b.close()
+
+
+def leading(lead, P, tiles, seed):
+    """`lead` empty rows, then rows with entries over `tiles` tiles of P."""
+    rng = np.random.default_rng(seed)
+    lens = [0] * lead
+    while sum(lens) < tiles * P - 30:
+        lens.append(int(rng.integers(1, 30)))
+    return lens
+
+
+# fewer empty rows than tiles, than lanes, and about their multiples: some waves
+# have no share of them, some a part of one
+LEADS = [1, 2, 63, 64, 65, 129, 1000, 4097]
+
+
+@pytest.mark.parametrize("tiles", [1, 3, 50, 131])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_leading_empty_rows_and_the_rows_behind_them(tiles, dtype):
+    """The leading empty rows are zeroed by shares and the rows behind them keep
+    their sums: on a handle, with the rows found inside the launch, and in a batch."""
+    cs = [cases.from_lengths(f"lead {lead}", leading(lead, 512, tiles, lead), n=5000, seed=lead)
+          for lead in LEADS]
+    print(f"[gpu] leading empty rows, {tiles} tiles, {np.dtype(dtype).name}", flush=True)
+    want = [km.segsum(c.row_ptr, c.col, c.val.astype(dtype), c.x.astype(dtype), S=8, TPW=1,
+                      alpha=0.5, dtype=dtype) for c in cs]
+    four = [km.segsum(c.row_ptr, c.col, c.val.astype(dtype), c.x.astype(dtype), S=8, TPW=4,
+                      alpha=0.5, dtype=dtype) for c in cs]
+    for c, w1, w4 in zip(cs, want, four):
+        v, x = c.val.astype(dtype), c.x.astype(dtype)
+        op, y = bhsparse_spmv(dtype), np.full(c.m, np.nan, dtype)
+        _lib.check(op.init_platform(0), "init_platform")
+        _lib.check(op.set_config(0, 8, 4, 1, 0), "set_config")
+        _lib.check(op.prepare_mem(c.m, c.n, c.nnz, c.row_ptr, c.col, v, x, y), "prepare_mem")
+        _lib.check(op.spmv(0.5), "spmv")
+        _lib.check(op.get_y(), "get_y")
+        op.close()
+        assert np.array_equal(y, w1), c.name
+        with DeviceArrays(np.asarray(c.row_ptr, np.int32), np.asarray(c.col, np.int32), v, x,
+                          np.full(c.m, np.nan, dtype)) as d:
+            _lib.check(call_noalloc(dtype, c.m, c.n, c.nnz, d.ptrs, 0.5), "spmv_noalloc")
+            assert np.array_equal(d.get(4, y), w4), c.name
+    mats = [matgen.CSR(c.m, c.n, c.row_ptr, c.col, c.val.astype(dtype), c.name) for c in cs]
+    ks = [(1, 2, 3, 16)[i % 4] for i in range(len(cs))]
+    b = batched.SpmvBatch(mats, ks, dtype)
+    b.set_x([np.repeat(c.x.astype(dtype)[:, None], k, 1) for c, k in zip(cs, ks)])
+    b.set_schedule(8, 1, 1, 0, 1, 0)
+    b.run(0.5)
+    for Y, w1, c in zip(b.y(), want, cs):
+        assert np.array_equal(Y, np.repeat(w1[:, None], Y.shape[1], 1)), c.name
+    b.close()
