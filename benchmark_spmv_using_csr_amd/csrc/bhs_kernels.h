@@ -960,7 +960,7 @@ struct TileShare {
 // point where the eight L2s meet (agent scope).
 struct ChainBuf {
     unsigned long long *pair;    // [NW * sizeof(T)/4] rows of two waves, by first wave
-    unsigned long long *count;   // [NW] longer rows: tag << 32 | arrivals, by first wave
+    unsigned long long *count;   // [NW] call << 32 | arrivals, by first wave
     void *own, *part;            // [NW] T: longer rows, the first wave's partial and the others'
     unsigned call;               // the call's number, 1 .. 2^31 - 1
 };
@@ -986,9 +986,10 @@ __device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first
     const int end = min(last - base, kWave - 1);
     if (last == e0) {
         // Two waves swap: lane h exchanges {tag, half h} for what lies there.
-        // The one that finds the other's first half finishes the row; if its
-        // other half is still on its way (it was swapped in the other order),
-        // it replaces this wave's own word shortly.
+        // The one that finds both of the other's halves finishes the row.  Were the
+        // halves swapped in different orders, each wave finds one; both then
+        // exchange the count, and the second to do so has the half that it
+        // lacks in memory: the other wave's exchanges are over.
         const unsigned tag = cb.call << 1 | (w == first ? 0u : 1u);   // the two sides differ
         unsigned half;
         if constexpr (H == 2) {
@@ -1002,12 +1003,22 @@ __device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first
         if (lane < H)
             got = __hip_atomic_exchange(p, (unsigned long long)tag << 32 | half, __ATOMIC_RELAXED,
                                         __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned other = tag ^ 1u;
-        if (__builtin_amdgcn_readfirstlane((unsigned)(got >> 32)) != other) return;
-        if (lane < H) {
-            for (int i = 0; i < (1 << 16) && (unsigned)(got >> 32) != other; ++i) got = agent_load(p);
-            agent_store(p, 0ull);
+        const bool found = (unsigned)(got >> 32) == (tag ^ 1u);   // no call's tag is 0
+        const uint64_t halves = ballot(found);
+        if (halves == 0) return;
+        if constexpr (H == 2) {
+            if (halves != 3) {
+                unsigned long long seen = 0ull;
+                if (lane == 0)
+                    seen = __hip_atomic_exchange(cb.count + first,
+                                                 (unsigned long long)cb.call << 32 | 1ull,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (__builtin_amdgcn_readfirstlane((unsigned)(seen >> 32)) != cb.call) return;
+                if (lane < H && !found) got = agent_load(p);
+                if (lane == 0) agent_store(cb.count + first, 0ull);
+            }
         }
+        if (lane < H) agent_store(p, 0ull);
         const unsigned lo = (unsigned)read_lane((int)(unsigned)got, 0);
         T o;
         if constexpr (H == 2) {
