@@ -1018,7 +1018,6 @@ __device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first
                 if (lane == 0) agent_store(cb.count + first, 0ull);
             }
         }
-        if (lane < H) agent_store(p, 0ull);
         const unsigned lo = (unsigned)read_lane((int)(unsigned)got, 0);
         T o;
         if constexpr (H == 2) {
@@ -1031,6 +1030,8 @@ __device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first
         T tot = w == first ? o : v;
         if (end == kWave - 1) tot = tot + T(0);       // as at a window's last entry
         if (lane == 0) y[row] = head + tot;
+        // last: a store ahead of a use of `got` would be waited for there
+        if (lane < H) agent_store(p, 0ull);
         return;
     }
     T *own = reinterpret_cast<T *>(cb.own), *part = reinterpret_cast<T *>(cb.part);
