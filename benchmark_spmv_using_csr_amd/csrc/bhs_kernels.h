@@ -175,12 +175,12 @@ struct BigTag {
 __device__ __forceinline__ int empty_run_end(const int *__restrict__ row_ptr, int lo, int v,
                                              int stop)
 {
-    int step = 64;
-    while (lo + step <= stop + 1 && row_ptr[lo + step] == v) {
+    unsigned step = 64;                      // steps by their length: lo + step may pass 2^31
+    while (step <= (unsigned)(stop + 1 - lo) && row_ptr[lo + step] == v) {
         lo += step;
         step *= 2;
     }
-    int hi = min(lo + step, stop + 1);
+    int hi = lo + (int)min(step, (unsigned)(stop + 1 - lo));
     if (row_ptr[hi] == v) return stop + 1;   // empty up to the tile's last row
     while (hi - lo > 1) {                    // row_ptr[lo] == v < row_ptr[hi]
         const int mid = lo + (hi - lo) / 2;

@@ -2,6 +2,8 @@
 (GPU): y must be the same bits for every tile shape it is built for, with the
 rows that cross logical waves finished inside the launch, and with the rows
 found inside it (the allocation-free entry point)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -9,7 +11,7 @@ import cases
 import kernel_model as km
 from benchmark_spmv_using_csr_amd import _lib, batched, matgen
 from benchmark_spmv_using_csr_amd.spmv import bhsparse_spmv
-from test_zz_no_alloc import DeviceArrays, call_noalloc
+from test_zz_no_alloc import DeviceArrays, call_noalloc, hip
 
 pytestmark = pytest.mark.gpu
 
@@ -253,3 +255,49 @@ def test_leading_empty_rows_and_the_rows_behind_them(tiles, dtype):
     for Y, w1, c in zip(b.y(), want, cs):
         assert np.array_equal(Y, np.repeat(w1[:, None], Y.shape[1], 1)), c.name
     b.close()
+
+
+@pytest.mark.parametrize("empty", [(1 << 30) + 7, 1_500_000_001])
+def test_more_empty_rows_than_half_the_index_range(empty):
+    """A run of over 2^30 empty rows between two groups of rows with entries: the
+    steps along it do not pass 2^31.  Whole numbers; y is read at both ends of the
+    run and at places inside."""
+    H = hip()
+    H.hipMemsetD32.argtypes = [C.c_void_p, C.c_int, C.c_size_t]
+    lens = [3] * 900
+    rp = np.cumsum([0] + lens).astype(np.int32)
+    m, half = empty + 1800, int(rp[-1])
+    nnz, n = 2 * half, 1000
+    rng = np.random.default_rng(1)
+    col = rng.integers(0, n, nnz).astype(np.int32)
+    val = rng.integers(-3, 4, nnz).astype(np.float32)
+    x = rng.integers(-3, 4, n).astype(np.float32)
+    want = np.add.reduceat(val * x[col], np.arange(0, nnz, 3))
+    ptr = {}
+    try:
+        for name, words in (("row_ptr", m + 1), ("y", m)):
+            ptr[name] = C.c_void_p()
+            assert H.hipMalloc(C.byref(ptr[name]), 4 * words) == 0
+        at = lambda name, i: C.c_void_p(ptr[name].value + 4 * i)
+        assert H.hipMemsetD32(ptr["row_ptr"], half, m + 1) == 0
+        assert H.hipMemsetD32(ptr["y"], 0x7fc00000, m) == 0            # NaN
+        assert H.hipMemcpy(at("row_ptr", 0), rp.ctypes.data_as(C.c_void_p), rp.nbytes, 1) == 0
+        tail = rp + np.int32(half)
+        assert H.hipMemcpy(at("row_ptr", m - 900), tail.ctypes.data_as(C.c_void_p), tail.nbytes,
+                           1) == 0
+        print(f"[gpu] {empty} empty rows in a row", flush=True)
+        with DeviceArrays(col, val, x) as d:
+            _lib.check(call_noalloc(np.float32, m, n, nnz,
+                                    [ptr["row_ptr"], *d.ptrs, ptr["y"]], 1.0), "spmv_noalloc")
+            assert H.hipDeviceSynchronize() == 0
+        def y(lo, hi):
+            out = np.empty(hi - lo, np.float32)
+            assert H.hipMemcpy(out.ctypes.data_as(C.c_void_p), at("y", lo), out.nbytes, 2) == 0
+            return out
+        assert np.array_equal(y(0, 900), want[:900])
+        assert np.array_equal(y(m - 900, m), want[900:])
+        for lo in (900, 5000, 1 << 29, 1 << 30, m // 2, m - 900 - 70_000):
+            assert not y(lo, min(lo + 70_000, m - 900)).any()
+    finally:
+        for p in ptr.values():
+            H.hipFree(p)
