@@ -721,7 +721,7 @@ int init_data(bhs_handle_t h, int m, int n, int nnz, const int *row_ptr, const i
     BHS_HIP(alloc_data(im, &im->d_val, sizeof(T) * (size_t)im->nnz_pad));
     BHS_HIP(alloc_data(im, &im->d_x, sizeof(T) * (size_t)std::max(n, 1)));
     BHS_HIP(alloc_data(im, &im->d_y, sizeof(T) * (size_t)std::max(m, 1)));
-    StageLease lease(im->stream, im->data_mode == BHS_MEMORY_DEVICE);
+    StageLease lease(im->stream, im->signal, im->data_mode == BHS_MEMORY_DEVICE);
     if (int rc = upload(lease, im->stream, im->d_row_ptr, row_ptr, sizeof(int) * ((size_t)m + 1)))
         return rc;
     // past the last nonzero: column 0, value 0
@@ -766,7 +766,8 @@ int set_x(bhs_handle_t h, const T *x)
     if (im->n > 0 && !x) return set_error(BHSPARSE_INVALID_ARGUMENT, "null x");
     BHS_HIP(hipSetDevice(im->device));
     const size_t bytes = sizeof(T) * (size_t)im->n;
-    StageLease lease(im->stream, im->n > 0 && im->data_mode == BHS_MEMORY_DEVICE && pageable(x));
+    StageLease lease(im->stream, im->signal,
+                     im->n > 0 && im->data_mode == BHS_MEMORY_DEVICE && pageable(x));
     if (lease) {
         if (int rc = lease.write(im->d_x, x, bytes)) return rc;
         return lease.finish();
@@ -1090,7 +1091,8 @@ int get_y_to(bhs_handle_t h, T *out)
     if (im->m > 0 && !out) return set_error(BHSPARSE_INVALID_ARGUMENT, "null y");
     BHS_HIP(hipSetDevice(im->device));
     const size_t bytes = sizeof(T) * (size_t)im->m;
-    StageLease lease(im->stream, im->m > 0 && im->data_mode == BHS_MEMORY_DEVICE && pageable(out));
+    StageLease lease(im->stream, im->signal,
+                     im->m > 0 && im->data_mode == BHS_MEMORY_DEVICE && pageable(out));
     if (lease)
         return lease.read(im->d_y, bytes, [&](size_t o, const char *p, size_t len) {
             copy_part(reinterpret_cast<char *>(out) + o, p, len, bytes >= kPastCaches);
