@@ -960,7 +960,7 @@ struct TileShare {
 // point where the eight L2s meet (agent scope).
 struct ChainBuf {
     unsigned long long *pair;    // [NW * sizeof(T)/4] rows of two waves, by first wave
-    unsigned long long *count;   // [NW] call << 32 | arrivals, by first wave
+    unsigned long long *count;   // [NW] call << 32 | arrivals, by first wave (of a row, of a group)
     void *own, *part;            // [NW] T: longer rows, the first wave's partial and the others'
     unsigned call;               // the call's number, 1 .. 2^31 - 1
 };
@@ -975,6 +975,26 @@ __device__ __forceinline__ void agent_store(U *p, U v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// Whether this is the last of n > 1 arrivals at `word`: the first one sets the tag
+// there, the rest add to it.
+__device__ __forceinline__ bool chain_arrive(unsigned long long *word, unsigned tag, int n)
+{
+    unsigned long long seen = 0ull;
+    while (seen >> 32 != tag)
+        if (__hip_atomic_compare_exchange_strong(word, &seen, (unsigned long long)tag << 32 | 1ull,
+                                                 __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+            return false;
+    return (unsigned)__hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT) == (unsigned)n - 1;
+}
+
+// Waves up to which a row's partials are counted at one word, and of a group
+// beyond.  A word takes an arrival every 28 ns or so: one row over 390 (800)
+// logical waves among 500,000 nonzeros, fp64, S = 4, T = 1, 14.6 (24.9) us a call
+// with one word, 8.0 (8.3) with groups, 9.7 (13.6) with calibrate_kernel.
+constexpr int kChainDirect = 64, kChainGroup = 32;
 
 // Wave w's partial v of `row`, whose nonzeros lie in waves first..last > first.
 template <typename T>
@@ -1035,23 +1055,27 @@ __device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first
         return;
     }
     T *own = reinterpret_cast<T *>(cb.own), *part = reinterpret_cast<T *>(cb.part);
-    const unsigned others = (unsigned)(last - first);
+    // Groups are counted at their first wave's word (no other row's: this one goes
+    // on past that wave, or the group is that wave alone and is not counted), and
+    // the groups at the row's pair word, free in a row of more than two waves.
     int complete = 0;
     if (lane == 0) {
         agent_store(w == first ? own + first : part + w, v);
         // the partial has arrived before the count says so
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        const unsigned long long tag = (unsigned long long)cb.call << 32;
-        unsigned long long seen = 0ull;
-        // the first to arrive sets the tag; the rest add to it
-        while (seen >> 32 != cb.call)
-            if (__hip_atomic_compare_exchange_strong(cb.count + first, &seen, tag | 1ull,
-                                                     __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT))
-                break;
-        if (seen >> 32 == cb.call)
-            complete = (unsigned)__hip_atomic_fetch_add(cb.count + first, 1ull, __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_AGENT) == others;
+        const int n = last - first + 1;
+        if (n <= kChainDirect) {
+            complete = chain_arrive(cb.count + first, cb.call, n);
+        } else {
+            const int g = w & ~(kChainGroup - 1), g0 = max(first, g);
+            const int ng = min(last, g + kChainGroup - 1) - g0 + 1;
+            complete = ng == 1 || chain_arrive(cb.count + g0, cb.call, ng);
+            if (complete) {
+                if (ng > 1) agent_store(cb.count + g0, 0ull);
+                complete = chain_arrive(cb.pair + (long long)first * H, cb.call << 1,
+                                        last / kChainGroup - first / kChainGroup + 1);
+            }
+        }
         asm volatile("" ::: "memory");
     }
     if (!__builtin_amdgcn_readfirstlane(complete)) return;
@@ -1077,7 +1101,8 @@ __device__ __forceinline__ void chain_add(const ChainBuf &cb, int row, int first
     if (lane == 0) {
         const T head = w == first ? v : agent_load(own + first);
         y[row] = head + tot;
-        agent_store(cb.count + first, 0ull);
+        agent_store(last - first < kChainDirect ? cb.count + first : cb.pair + (long long)first * H,
+                    0ull);
     }
 }
 

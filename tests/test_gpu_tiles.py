@@ -301,3 +301,56 @@ def test_more_empty_rows_than_half_the_index_range(empty):
     finally:
         for p in ptr.values():
             H.hipFree(p)
+
+
+@pytest.mark.parametrize("T", [1, 4])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_long_rows_counted_by_groups(T, dtype):
+    """Rows over 63 to 300 logical waves whose first and last waves lie on, before
+    and behind the ends of groups of 32, one behind the other (the last wave of
+    one is the first of the next) and with short ones between."""
+    PW, lens, at = 64 * 4 * T, [], 0
+
+    def to(wave, inside):                      # a row up to `inside` nonzeros into a wave
+        nonlocal at
+        lens.append(wave * PW + inside - at)
+        at = wave * PW + inside
+
+    for wave, inside in [(0, 5), (63, 9), (64, 3), (127, 7), (128, 1), (193, 2), (256, 4), (321, PW),
+                         (352, 11), (417, 8), (482, 6), (546, PW), (578, 1), (578, 40), (672, 1),
+                         (735, 5), (736, 5), (1036, 9)]:
+        to(wave, inside)
+    lens += [3, 0, 2]
+    c = cases.from_lengths("groups", lens, n=5000, seed=T)
+    v, x = c.val.astype(dtype), c.x.astype(dtype)
+    op, y = bhsparse_spmv(dtype), np.zeros(c.m, dtype)
+    _lib.check(op.init_platform(0), "init_platform")
+    _lib.check(op.set_config(0, 4, 1, T, 0), "set_config")
+    _lib.check(op.prepare_mem(c.m, c.n, c.nnz, c.row_ptr, c.col, v, x, y), "prepare_mem")
+    print(f"[gpu] long rows by groups T={T} {np.dtype(dtype).name} nnz={c.nnz}", flush=True)
+    ym = km.segsum(c.row_ptr, c.col, v, x, S=4, TPW=T, dtype=dtype)
+    for _ in range(3):
+        _lib.check(op.spmv(1.0), "spmv")
+        _lib.check(op.get_y(), "get_y")
+        assert np.array_equal(y, ym), np.flatnonzero(y != ym)
+    op.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_long_rows_found_inside_the_launch(dtype):
+    """Rows over 70 to 2,500 logical waves of the default tile through the
+    allocation-free entry point; whole numbers."""
+    lens = [4, 70 * 2048 + 3, 0, 9, 700 * 2048, 1, 2500 * 2048 + 77, 5]
+    row_ptr = np.r_[0, np.cumsum(lens)].astype(np.int32)
+    m, n, nnz = len(lens), 1000, int(row_ptr[-1])
+    col = np.arange(nnz, dtype=np.int32) % n
+    x = (np.arange(n) % 7 - 3).astype(dtype)
+    val = np.ones(nnz, dtype)
+    print(f"[gpu] {nnz} nonzeros in {m} rows {np.dtype(dtype).name}", flush=True)
+    sums = np.r_[0, np.cumsum(x.astype(np.int64)[col])]
+    y0 = np.full(m, np.nan, dtype)
+    with DeviceArrays(row_ptr, col, val, x, y0) as d:
+        for _ in range(2):
+            _lib.check(call_noalloc(dtype, m, n, nnz, d.ptrs, 2.0), "spmv_noalloc")
+            y = d.get(4, y0)
+            assert np.array_equal(y.astype(np.int64), 2 * (sums[row_ptr[1:]] - sums[row_ptr[:-1]]))
