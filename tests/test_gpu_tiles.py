@@ -354,3 +354,47 @@ def test_long_rows_found_inside_the_launch(dtype):
             _lib.check(call_noalloc(dtype, m, n, nnz, d.ptrs, 2.0), "spmv_noalloc")
             y = d.get(4, y0)
             assert np.array_equal(y.astype(np.int64), 2 * (sums[row_ptr[1:]] - sums[row_ptr[:-1]]))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_runs_of_empty_rows_at_every_alignment(dtype):
+    """Runs of 128 to 1,500 empty rows that start and end at every offset from 16
+    bytes, y itself at each of them; the values before and behind y stay."""
+    rng = np.random.default_rng(5)
+    lens = []
+    for run in [128, 129, 130, 131, 255, 256, 257, 700, 1001, 1002, 1003, 1500]:
+        lens += list(rng.integers(1, 4, int(rng.integers(1, 6)))) + [0] * run
+    lens += [2, 1]
+    c = cases.from_lengths("runs", lens, n=3000, seed=6)
+    v, x = c.val.astype(dtype), c.x.astype(dtype)
+    want = km.segsum(c.row_ptr, c.col, v, x, S=8, TPW=4, dtype=dtype)
+    print(f"[gpu] runs of empty rows {np.dtype(dtype).name}", flush=True)
+    room = np.full(c.m + 16, 7, dtype)
+    for off in range(16 // room.itemsize):
+        with DeviceArrays(np.asarray(c.row_ptr, np.int32), np.asarray(c.col, np.int32), v, x,
+                          room) as d:
+            y = C.c_void_p(d.ptrs[4].value + (4 + off) * room.itemsize)
+            _lib.check(call_noalloc(dtype, c.m, c.n, c.nnz, [*d.ptrs[:4], y], 1.0), "spmv_noalloc")
+            got = d.get(4, room)
+        assert np.array_equal(got[4 + off:4 + off + c.m], want), off
+        assert np.all(got[:4 + off] == 7) and np.all(got[4 + off + c.m:] == 7)
+    for tile in [(0, 8, 4, 1, 0), (0, 4, 1, 16, 0)]:          # a wave per tile; the tile loop
+        op, y = bhsparse_spmv(dtype), np.full(c.m, np.nan, dtype)
+        _lib.check(op.init_platform(0), "init_platform")
+        _lib.check(op.set_config(*tile), "set_config")
+        _lib.check(op.prepare_mem(c.m, c.n, c.nnz, c.row_ptr, c.col, v, x, y), "prepare_mem")
+        _lib.check(op.spmv(1.0), "spmv")
+        _lib.check(op.get_y(), "get_y")
+        op.close()
+        assert np.array_equal(y, km.segsum(c.row_ptr, c.col, v, x, S=tile[1], TPW=tile[3],
+                                           dtype=dtype)), tile
+    A = matgen.CSR(c.m, c.n, c.row_ptr, c.col, v, c.name)
+    for T in (4, 16):                                         # a wave per tile; the tile loop
+        b = batched.SpmvBatch([A] * 4, [1, 2, 3, 16], dtype)
+        b.set_schedule(8, T, 1, 0, 1, 0)
+        b.set_x([np.repeat(x[:, None], k, 1) for k in (1, 2, 3, 16)])
+        b.run(1.0)
+        b.run_plain(1.0)
+        for Y, P in zip(b.y(), b.y(plain=True)):
+            assert np.array_equal(Y, P) and not np.isnan(Y).any()
+        b.close()
