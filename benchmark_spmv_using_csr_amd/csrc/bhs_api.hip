@@ -563,6 +563,11 @@ size_t tile_lds_bytes(int S, int waves)
 //    uniform rows 10.7 / 9.1, band of 41 8.4 / 6.1, power law with one row
 //    over 390 waves 12.3 / 13.3; 2M (7.8k), power law 22.2 / 22.7.
 //  * fp32, S = 4 (2 KB of A a wave), T = 4, Laplacian 160^3: 63.9 / 70.8 warm.
+//  * Rows of more than a logical wave on average: nearly every wave hands two rows
+//    over, one after the other.  Fused / loop, T = 1, rows of 1.8 to 61 waves, 150k to
+//    2M nonzeros: 1.05 to 1.30; rows of 1.3 waves 0.94 to 1.09, of half a wave 0.60 to
+//    0.90.  T = 4, S = 8: 600k nonzeros (290 waves) 0.71 to 0.93; 8M (3.9k) fused 0.96
+//    to 1.06, not fused 0.94 to 1.00.
 //  * T > 1 with up to 24 logical waves (49,000 nonzeros at the default tile)
 //    stays on the loop, 13 us against 5.6: the fixed default tile is the yardstick
 //    of the tuner's speedup (at least 1.2 over its test set: 1.10 without this
@@ -579,7 +584,9 @@ SegsumKernel pick_kernel(const Impl<T> *im, long long NW)
         return kWaveLoop;
     if (tile_lds_bytes<T>(S, tile_block_waves(c)) > im->dev_lds) return kWaveLoop;
     if (TPW > 1 && NW <= 24) return kWaveLoop;
-    if (NW <= (TPW == 1 || S == 4 ? 4096 : 16384)) return kTilePerWaveFused;
+    const bool long_rows = im->nnz > 64LL * S * TPW * im->m;
+    if (long_rows && TPW == 1) return kWaveLoop;
+    if (NW <= (long_rows ? 1024 : TPW == 1 || S == 4 ? 4096 : 16384)) return kTilePerWaveFused;
     return TPW == 1 || S * sizeof(T) < 32 ? kWaveLoop : kTilePerWave;
 }
 

@@ -63,3 +63,32 @@ def test_a_plain_class_after_csr_vector(dtype, waves):
         _lib.check(op.get_y(), "get_y")
         assert np.array_equal(y, fresh)
     op.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_long_rows_on_average_leave_the_fused_kernel(dtype):
+    """The line lies at a mean row of one logical wave: at T = 1 the loop and a
+    calibration beyond it, at T = 4 from 1,024 logical waves on; y is the same bits
+    on both sides (one empty row more or less does not move a sum)."""
+    rng = np.random.default_rng(2)
+    for tile, length, rows, beyond in [((0, 8, 4, 1, 0), 512, 700, 2), ((0, 8, 4, 4, 0), 2048, 300, 1),
+                                       ((0, 8, 4, 4, 0), 2048, 1100, 2)]:
+        nnz, n = length * rows, 50_000
+        cuts = np.sort(rng.choice(nnz, rows - 2, False))         # rows - 1 rows of any length
+        row_ptr = np.r_[0, cuts, nnz].astype(np.int32)
+        col, val = rng.integers(0, n, nnz).astype(np.int32), rng.uniform(-1, 1, nnz).astype(dtype)
+        x, got = rng.uniform(-1, 1, n).astype(dtype), []
+        for extra, kernels in ((0, beyond), (1, 1)):             # rows - 1, then rows of them
+            rp = np.r_[row_ptr, np.full(extra, nnz, np.int32)].astype(np.int32)
+            op, y = bhsparse_spmv(dtype), np.full(len(rp) - 1, np.nan, dtype)
+            _lib.check(op.init_platform(0), "init_platform")
+            _lib.check(op.set_config(*tile), "set_config")
+            _lib.check(op.prepare_mem(len(rp) - 1, n, nnz, rp, col, val, x, y), "prepare_mem")
+            print(f"[gpu] {tile} {rows - 1 + extra} rows, {nnz} nonzeros", flush=True)
+            assert kernels_of_a_call(op) == kernels
+            for _ in range(2):
+                _lib.check(op.spmv(1.0), "spmv")
+            _lib.check(op.get_y(), "get_y")
+            op.close()
+            got.append(y[:rows - 1])
+        assert np.array_equal(*got)
