@@ -398,3 +398,92 @@ def test_runs_of_empty_rows_at_every_alignment(dtype):
         for Y, P in zip(b.y(), b.y(plain=True)):
             assert np.array_equal(Y, P) and not np.isnan(Y).any()
         b.close()
+
+
+def rows_over_waves(PW, waves, lead, seed):
+    """Rows over 3, 64, 65 and 200 logical waves, rows that end on a wave's end and
+    one to either side, runs of empty rows at wave ends and inside, `lead` empty rows
+    first; the mean row is longer than a logical wave."""
+    rng = np.random.default_rng(seed)
+    lens, at = [0] * lead, 0
+
+    def to(n):
+        nonlocal at
+        lens.append(n)
+        at += n
+
+    long = [3 * PW + 7, 64 * PW, 65 * PW - 5, 200 * PW + 1, 2 * PW]
+    while at < waves * PW:
+        left = PW - at % PW
+        pick = rng.integers(0, 7)
+        if pick == 0 and long:
+            to(long.pop())
+        elif pick == 1:
+            to(left)
+            lens += [0] * int(rng.integers(0, 4))
+        elif pick == 2:
+            to(left + PW)
+            lens += [0] * int(rng.choice([0, 70, 140]) if len(lens) < 300 else 0)
+        elif pick == 3:
+            to(left + 1)
+        elif pick == 4:
+            to(left + 2 * PW - 1)
+            to(2)
+        else:
+            to(left + int(rng.integers(1, 4 * PW)))
+    for n in long:
+        to(n)
+    return lens + [0] * 3
+
+
+@pytest.mark.parametrize("S,T", [(4, 2), (4, 8), (8, 2), (8, 4), (16, 2), (16, 4)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_rows_left_to_the_calibration(S, T, dtype):
+    """One wave per tile without the fused end: rows that pass through whole logical
+    waves, and leading empty rows.  Whole numbers, so the sums are exact."""
+    from test_gpu_choice import kernels_of_a_call
+    for lead in (0, 1, 65, 500):
+        lens = rows_over_waves(64 * S * T, 1300, lead, 10 * S + T + lead)
+        row_ptr = np.r_[0, np.cumsum(lens)].astype(np.int32)
+        m, n, nnz = len(lens), 3000, int(row_ptr[-1])
+        assert nnz > 64 * S * T * m
+        rng = np.random.default_rng(S + T)
+        col = rng.integers(0, n, nnz).astype(np.int32)
+        val, x = rng.integers(-3, 4, nnz), rng.integers(-3, 4, n)
+        sums = np.r_[0, np.cumsum(val * x[col])]
+        op, y = bhsparse_spmv(dtype), np.full(m, np.nan, dtype)
+        _lib.check(op.init_platform(0), "init_platform")
+        _lib.check(op.set_config(0, S, 4, T, 0), "set_config")
+        _lib.check(op.prepare_mem(m, n, nnz, row_ptr, col, val.astype(dtype), x.astype(dtype), y),
+                   "prepare_mem")
+        print(f"[gpu] left to the calibration: S={S} T={T} lead={lead} nnz={nnz} "
+              f"{np.dtype(dtype).name}", flush=True)
+        assert kernels_of_a_call(op) == 2
+        for alpha in (1.0, -2.0):
+            _lib.check(op.spmv(alpha), "spmv")
+            _lib.check(op.get_y(), "get_y")
+            assert np.array_equal(y, alpha * (sums[row_ptr[1:]] - sums[row_ptr[:-1]]))
+        op.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_rows_left_to_the_calibration_bit_for_bit(dtype):
+    """The same kind of rows at the default tile against the allocation-free entry
+    point, whose launch finishes them itself."""
+    from test_gpu_choice import kernels_of_a_call
+    lens = rows_over_waves(2048, 1300, 65, 1)
+    row_ptr = np.r_[0, np.cumsum(lens)].astype(np.int32)
+    m, n, nnz = len(lens), 40_000, int(row_ptr[-1])
+    rng = np.random.default_rng(2)
+    col = rng.integers(0, n, nnz).astype(np.int32)
+    val, x = rng.uniform(-1, 1, nnz).astype(dtype), rng.uniform(-1, 1, n).astype(dtype)
+    op, y = bhsparse_spmv(dtype), np.full(m, np.nan, dtype)
+    _lib.check(op.init_platform(0), "init_platform")
+    _lib.check(op.prepare_mem(m, n, nnz, row_ptr, col, val, x, y), "prepare_mem")
+    assert kernels_of_a_call(op) == 2
+    _lib.check(op.spmv(0.75), "spmv")
+    _lib.check(op.get_y(), "get_y")
+    op.close()
+    with DeviceArrays(row_ptr, col, val, x, np.full(m, np.nan, dtype)) as d:
+        _lib.check(call_noalloc(dtype, m, n, nnz, d.ptrs, 0.75), "spmv_noalloc")
+        assert np.array_equal(d.get(4, y), y)
