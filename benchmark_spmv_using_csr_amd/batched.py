@@ -106,8 +106,10 @@ class SpmvBatch:
 
 # Candidate schedules for the batch autotuner: (S, T, waves/block, grid, order,
 # x_stage).  The x-staged ones run on fp64 batches only (the autotuner skips
-# them elsewhere).
-SCHEDULES = [(S, T, wpb, 0, 1, 0) for S in (4, 8) for T in (1, 4, 16) for wpb in (1, 4)] + \
+# them elsewhere).  waves/block shapes only the launches of T > 8 and of the
+# x-staged ones, so the others are listed with one value of it.
+SCHEDULES = [(S, T, 4, 0, 1, 0) for S in (4, 8) for T in (1, 4)] + \
+            [(S, 16, wpb, 0, 1, 0) for S in (4, 8) for wpb in (1, 4)] + \
             [(4, T, wpb, 0, 1, 0) for T in (32, 64) for wpb in (1, 4)] + [(8, 4, 4, 0, 0, 0)] + \
             [(4, T, 1, 0, 1, xs) for xs in (2, 4) for T in (8, 16, 32)]
 
