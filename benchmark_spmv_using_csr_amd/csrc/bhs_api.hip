@@ -611,6 +611,7 @@ int ensure_analysis(Impl<T> *im)
         im->kernel = pick_kernel(im, im->NW);   // csr-vector and plain classes share a partition
         return BHSPARSE_SUCCESS;
     }
+    im->an_P = 0;                // none until this one is finished
     if (layout > 0 && im->m > 0)
         if (int rc = build_panels(im, layout)) return rc;
     const Layout<T> L = active_layout(im);
@@ -618,6 +619,7 @@ int ensure_analysis(Impl<T> *im)
     const long long NW = (NP + TPW - 1) / TPW;
     if (NP + 1 > im->tile_cap) {
         free_ptr(im->d_tile_row);
+        im->tile_cap = 0;
         BHS_HIP(hipMalloc(&im->d_tile_row, sizeof(int) * (size_t)(NP + 1)));
         im->tile_cap = (int)(NP + 1);
     }
