@@ -184,8 +184,8 @@ def run_batched():
                      "traffic": load_traffic("batched_256mat_f64_traffic.json", sched,
                                              key="schedule"),
                      "definition": "effective bytes of the batch (A once, x and y per "
-                                   "right-hand side) / median graph replay (queue reset, "
-                                   "batched_kernel, calibration)"},
+                                   "right-hand side) / median graph replay (the batched "
+                                   "kernel and its calibration)"},
         "schedule": {"items_per_lane": sched[0], "tiles_per_wave": sched[1],
                      "waves_per_block": sched[2], "grid_blocks": sched[3],
                      "order": "matrix" if sched[4] == 0 else "most work first",
@@ -364,7 +364,7 @@ def main():
     med_total = median(r["ms_total"])
     # the main kernel's duration: the mean interval between the start and end
     # events attached to its dispatch (hipExtLaunchKernelGGL), on the stream it
-    # runs on.  It agrees with rocprofv3's kernel-trace average for the same
+    # runs on, or around it where it is the call's only kernel.  It agrees with rocprofv3's kernel-trace average for the same
     # kernel (profiles/); the fixed cost of an empty interval between the same
     # events is reported beside it, not subtracted
     ev_ms = median(r["event_overhead"])
@@ -412,7 +412,8 @@ def main():
             "frac": round(achieved / HBM_PEAK_GBPS, 4),
             "traffic": traffic,
             "definition": "achieved = the call's algorithmic bytes / the main kernel's mean "
-                          "duration (dispatch-attached HIP events); whole_call_frac uses the "
+                          "duration (HIP events attached to its dispatch, or around it where "
+                          "it is the call's only kernel); whole_call_frac uses the "
                           "median whole call (every kernel of it) instead",
             "whole_call_frac": round(value / HBM_PEAK_GBPS, 4),
             "kernel": kname,

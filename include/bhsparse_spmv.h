@@ -184,7 +184,8 @@ int bhs_s_get_stats(bhs_handle_t h, bhs_spmv_stats *out);
  * flush_bytes > 0, a buffer of that size is written before every call (outside
  * the events) so caches start cold.  ms_total[i] = whole call; ms_main[i] =
  * main kernel only, from a second pass of calls with events attached to that
- * kernel's dispatch (both may be NULL). */
+ * kernel's dispatch, or, where the call is that one kernel, recorded around it
+ * as for a whole call (both may be NULL). */
 int bhs_s_bench(bhs_handle_t h, float alpha, int warmup, int reps, long long flush_bytes,
                 double *ms_total, double *ms_main);
 /* GPU reduction over row_ptr/col: 8 row-length features (m, nnz, mean, var,
