@@ -364,9 +364,10 @@ def main():
     med_total = median(r["ms_total"])
     # the main kernel's duration: the mean interval between the start and end
     # events attached to its dispatch (hipExtLaunchKernelGGL), on the stream it
-    # runs on, or around it where it is the call's only kernel.  It agrees with rocprofv3's kernel-trace average for the same
-    # kernel (profiles/); the fixed cost of an empty interval between the same
-    # events is reported beside it, not subtracted
+    # runs on, or around it where it is the call's only kernel.  It agrees with
+    # rocprofv3's kernel-trace average for the same kernel (profiles/); the fixed
+    # cost of an empty interval between the same events is reported beside it,
+    # not subtracted
     ev_ms = median(r["event_overhead"])
     mean_main = float(np.mean(r["ms_main"]))
     value = b / (med_total * 1e-3) / 1e9

@@ -71,7 +71,8 @@ def test_long_rows_on_average_leave_the_fused_kernel(dtype):
     calibration beyond it, at T = 4 from 1,024 logical waves on; y is the same bits
     on both sides (one empty row more or less does not move a sum)."""
     rng = np.random.default_rng(2)
-    for tile, length, rows, beyond in [((0, 8, 4, 1, 0), 512, 700, 2), ((0, 8, 4, 4, 0), 2048, 300, 1),
+    for tile, length, rows, beyond in [((0, 8, 4, 1, 0), 512, 700, 2),
+                                       ((0, 8, 4, 4, 0), 2048, 300, 1),
                                        ((0, 8, 4, 4, 0), 2048, 1100, 2)]:
         nnz, n = length * rows, 50_000
         cuts = np.sort(rng.choice(nnz, rows - 2, False))         # rows - 1 rows of any length

@@ -20,7 +20,7 @@ void refuse_malloc(int n) { refuse = n; }
 int hipMalloc(void **p, size_t n)
 {
     static int (*real)(void **, size_t);
-    if (!real) real = (int (*)(void **, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
+    if (!real) *(void **)&real = dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
     if (refuse && --refuse == 0) { *p = NULL; return 2; }     /* hipErrorOutOfMemory */
     return real(p, n);
 }
